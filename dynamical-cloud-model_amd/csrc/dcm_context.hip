@@ -367,6 +367,9 @@ int dcm_context_create(int ip, int jp, int kp, const double *dx, const double *d
         ae[i] = 1.0 / (dx[i - 1] * dxn[i]);
         aw[i] = 1.0 / (dx[i - 1] * dxn[i - 1]);
     }
+    c->uniform_x = true;
+    for (int i = 2; i <= ip; ++i)
+        c->uniform_x = c->uniform_x && ae[i] == ae[1] && aw[i] == aw[1];
     for (int j = 1; j <= jp; ++j) {
         an[j] = 1.0 / (dy[j - 1] * dyn[j]);
         as[j] = 1.0 / (dy[j - 1] * dyn[j - 1]);
@@ -464,12 +467,12 @@ int dcm_context_create(int ip, int jp, int kp, const double *dx, const double *d
         return DCM_OUT_OF_MEMORY;
     }
     c->hscal = (double *)p;
-    if (hipMalloc(&p, 2 * sizeof(SolverScalars)) != hipSuccess) {
+    if (hipMalloc(&p, 5 * sizeof(SolverScalars)) != hipSuccess) {
         set_error("hipMalloc failed");
         return DCM_OUT_OF_MEMORY;
     }
     c->solver = (SolverScalars *)p;
-    (void)hipMemset(c->solver, 0, 2 * sizeof(SolverScalars));
+    (void)hipMemset(c->solver, 0, 5 * sizeof(SolverScalars));
     if (hipHostMalloc(&p, 2 * sizeof(SolverScalars), hipHostMallocDefault) != hipSuccess) {
         set_error("hipHostMalloc failed");
         return DCM_OUT_OF_MEMORY;
@@ -531,6 +534,8 @@ int dcm_context_destroy(dcm_ctx *c) {
         (void)hipEventDestroy(p.second.second);
     }
     for (auto e : c->event_pool) (void)hipEventDestroy(e);
+    for (hipEvent_t e : c->poll_event)
+        if (e) (void)hipEventDestroy(e);
     if (c->iter_graph) (void)hipGraphExecDestroy(c->iter_graph);
     if (c->chunk_graph) (void)hipGraphExecDestroy(c->chunk_graph);
     c->solve_tables.release();

@@ -179,6 +179,7 @@ struct dcm_ctx {
     // scratch of the batched FP32 MPDATA: mp32_count padded FP32 fields
     float *mp32 = nullptr;
     size_t mp32_count = 0;
+    bool uniform_x = false;          // the x coefficients are the same in every plane
     std::vector<double> h_dx, h_dy, h_dz, h_dxn, h_dyn, h_dzn, h_rhoa, h_rhoan;
     // reduction scratch
     double *partials = nullptr;      // per-block partial sums (several slots)
@@ -187,7 +188,7 @@ struct dcm_ctx {
     size_t partials_adv_cap = 0;
     double *dscal = nullptr;         // generic device scalars (64 doubles)
     double *hscal = nullptr;         // pinned host mirror (64 doubles)
-    dcm::SolverScalars *solver = nullptr;   // device
+    dcm::SolverScalars *solver = nullptr;   // device (5: the solve's state, and the fused kernels' slots)
     dcm::SolverScalars *h_solver = nullptr; // pinned host
     // lazily allocated work fields (FP64 padded) and compact solver vectors
     std::vector<double *> work64;
@@ -228,6 +229,8 @@ struct dcm_ctx {
     dcm::DeviceScratch solve_tables, flags;
     int *h_flags = nullptr;
     size_t h_flags_cap = 0;
+    // the fused small-system solve: the flags of its last two chunks are there
+    hipEvent_t poll_event[2] = {nullptr, nullptr};
     // the stream is borrowed (an ensemble's), not owned
     bool borrowed_stream = false;
     std::unordered_map<const void *, dcm::Mirror> mirrors;

@@ -910,15 +910,15 @@ __global__ __launch_bounds__(256) void k_matvec_dot_b(IterArgs A, int xi, int ai
 }
 
 // x = x + alf*p + omg*cs; r = s - omg*t; partial sums of <r,r>, <r,cr>
-// (dynamics.f90:419-423), all compact vectors, grid-stride
-template <typename R>
+// (dynamics.f90:419-423), all compact vectors, grid-stride; SC: a pointer to
+// the scalars, in global memory or LDS (the caller has tested that the
+// iteration goes on)
+template <typename R, typename SC>
 __device__ __forceinline__ void update_body(gp<R> __restrict__ x, gp<const R> __restrict__ p,
                                             gp<const R> __restrict__ cs, gp<const R> __restrict__ s,
                                             gp<const R> __restrict__ t, gp<const R> __restrict__ cr,
                                             gp<R> __restrict__ r, int n, int nbu,
-                                            gp<const SolverScalars> __restrict__ sc,
-                                            double *partials, int lb) {
-    if (halted(sc)) return;
+                                            SC sc, double *partials, int lb) {
     const int stride = nbu;
     const R alf = (R)sc->alf, omg = (R)sc->omg;
     // the correction of a mixed inner solve (guard set) starts at zero: not
@@ -943,6 +943,7 @@ __global__ __launch_bounds__(256) void k_update(R *__restrict__ x, const R *__re
                                                 int n, int nbu,
                                                 const SolverScalars *__restrict__ sc,
                                                 double *partials) {
+    if (halted(sc)) return;
     update_body<R>(glob(x), glob(p), glob(cs), glob(s), glob(t), glob(cr), glob(r), n, nbu,
                    glob(sc), partials, (int)blockIdx.x);
 }
@@ -1016,11 +1017,443 @@ template <typename R>
 __global__ __launch_bounds__(256) void k_update_b(IterArgs A) {
     int lb;
     const IterMember &M = member_u(A, lb);
+    if (halted(M.sc)) return;
     update_body<R>(glob((R *)M.V[VX]), glob((const R *)M.V[VP]),
                    glob((const R *)M.V[VCS]), glob((const R *)M.V[VS]),
                    glob((const R *)M.V[VT]), glob((const R *)M.V[VCR]),
                    glob((R *)M.V[VR]), M.n, M.nbu, glob((const SolverScalars *)M.sc),
                    M.part, lb);
+}
+
+// ---------------------------------------------------------------------------
+// Small systems: the iteration in three kernels (seven with the default
+// twelve Chebyshev divisions) instead of 14 (29).
+//
+// Up to about a million cells every pass of the iteration above is bound by
+// its launch (3 to 7 us each against 1 to 3 us of memory time), so a system
+// that small runs whole groups of passes per launch.  A block owns a tile of
+// 8 x jt columns (the marching tiles of those columns, every level), reads
+// its right-hand side with a halo as wide as the group has stencil passes,
+// keeps the iterate in registers and LDS and lets the valid region shrink by
+// one column a pass: the halo columns are recomputed (2 to 6 times the work,
+// which the idle CUs of a small grid have to spare) instead of exchanged.
+// Measured per FP64 step: 1x101x120 6.8 -> 2.7 ms, 64^3 7.5 -> 4.7 ms; of a
+// 22 us launch at 64^3, the loads take 2 us, the folds and scalars 2, the
+// sweeps 8 (bound by FP64 issue), the sums and stores 4.  The one-block reductions go too: each kernel's blocks all fold
+// the partial sums of the kernel before it (the same tree, so the same bits)
+// and apply the scalar recurrence themselves; block 0 stores the result for
+// the next kernel in a slot that no block of this launch reads.
+//   A: fold <r,r>,<r,cr>; t = r - bet*(omg*v1), sweeps, p, v1 = A p, <cr,v1>
+//   C: fold <cr,v1>; s = r - alf*v1, sweeps, cs, t = A cs, <t,t>, <t,s>
+//   U: fold <t,t>,<t,s>; x, r, <r,r>, <r,cr>
+// Every value and every partial sum is the one of the kernels above, bit for
+// bit (a batched solve of the same system runs those).  p and v1 alternate
+// between two buffers, because a block reads its neighbours' old values.
+// ---------------------------------------------------------------------------
+
+// x / b by Markstein's theorem (IBM J. Res. Dev. 34, 1990): with y = 1/b
+// correctly rounded, one residual step makes x*y faithful and a second one
+// is the correctly rounded quotient, the IEEE one, in 5 operations instead
+// of a division's dozen.  The theorem needs exact residuals: quotients near
+// the ends of the exponent range take the division.
+__device__ __forceinline__ double div_by(double x, double b, double y) {
+    const double q0 = x * y;
+    const double q1 = __builtin_fma(__builtin_fma(-b, q0, x), y, q0);
+    const double q2 = __builtin_fma(__builtin_fma(-b, q1, x), y, q1);
+    const double ax = fabs(x);
+    if (__builtin_expect(!((ax >= 0x1p-900 && ax <= 0x1p900) || x == 0.0), 0)) return x / b;
+    return q2;
+}
+__device__ __forceinline__ float div_by(float x, float, float y) { return x * y; }
+__device__ __forceinline__ double recip(double b) { return 1.0 / b; }
+__device__ __forceinline__ float recip(float b) { return __builtin_amdgcn_rcpf(b); }
+
+// reduce_slot_1024 of NS <= 2 slots of n <= 1024 values each (slot s at
+// p + s*n) by a block of any whole number of waves: the sums in every
+// thread.  red: 2048 doubles of LDS.  Split in two, so that a kernel issues
+// its other loads between them.  The tree's pairs above n add zeros and are
+// left out.
+template <int NS>
+__device__ __forceinline__ void fold_load(const double *p, int n, double *red) {
+    const int w = n <= 64 ? 64 : (n <= 128 ? 128 : (n <= 256 ? 256 : (n <= 512 ? 512 : 1024)));
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+        for (int e = threadIdx.x; e < w; e += blockDim.x)
+            red[s * 1024 + e] = e < n ? 0.0 + p[s * n + e] : 0.0;
+}
+template <int NS>
+__device__ __forceinline__ void fold_sum(int n, double *red, double (&out)[NS]) {
+    const int t = threadIdx.x, nt = blockDim.x;
+    int w = n <= 64 ? 64 : (n <= 128 ? 128 : (n <= 256 ? 256 : (n <= 512 ? 512 : 1024)));
+    __syncthreads();
+    for (w >>= 1; w >= 64; w >>= 1) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+            for (int e = t; e < w; e += nt) red[s * 1024 + e] += red[s * 1024 + e + w];
+        __syncthreads();
+    }
+    // every wave sums the last 64 for itself
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        out[s] = wave_sum(red[s * 1024 + (t & 63)]);  // (lane 0's is the sum)
+    }
+}
+
+// Tile and box of a fused kernel: own columns TI x TJ, hi/hj columns of halo
+// (none along an axis that the tile covers whole).  A thread owns NP (j,k)
+// positions of the box and all their i planes, in registers: its i
+// neighbours are its own values, the j and k neighbours come from LDS.  The
+// grid is uniform along x (a rule of the launch), so a position's
+// coefficients, a_p and 1/a_p are the same in every plane.
+struct BoxGeo {
+    int TI, TJ, BI, BJ, hi, hj, nti, ntj;
+};
+constexpr int kGroup = 4;        // stencil passes per launch
+constexpr int kBoxPlanes = 16;   // 8 own planes and kGroup of halo either side
+
+template <typename R> struct SweepArgs {
+    const R *r, *v1;        // MODE 0, 1: the right-hand side's operands
+    const R *t, *s;         // MODE 2: right-hand side and iterate
+    R *t_out, *s_out;       // own cells (t_out may be null)
+    const R *p_old;         // non-null: s_out = s + bet*p_old
+    const R *dot;           // non-null: y = A s_out, partial sums with dot
+    R *y_out;
+    int nsw, two;           // sweeps; two: <y,y>, <y,dot> instead of <dot,y>
+    R w[kGroup + 1];        // relaxation of s0 and of each sweep (W)
+    MG m;
+    BoxGeo b;
+    CoefPack cp;
+    const SolverScalars *in;  // the scalars, before the fold of this kernel
+    SolverScalars *out;       // after it (block 0)
+    const double *pin;        // partial sums to fold (MODE 0: null on the first iteration)
+    int npin;
+    double *pout;
+};
+
+// LDS of a fused kernel: the box as [position][plane], a position's planes
+// padded to an odd stride (consecutive lanes in different banks, a plane an
+// immediate offset); the folds and the threads' sums share that space
+template <typename R> static size_t sweep_lds(const BoxGeo &b, const MG &m) {
+    const int stride = b.BI == 1 ? 1 : kBoxPlanes + 1;
+    const size_t box = (size_t)stride * b.BJ * m.kp * sizeof(R);
+    const size_t sums = 2 * 256 * (size_t)m.nkb * sizeof(double), fold = 2048 * sizeof(double);
+    return std::max(box, std::max(sums, fold));
+}
+
+static_assert(sizeof(SolverScalars) % 8 == 0, "SolverScalars is copied in 8-byte words");
+
+// NT: threads at most; NB: planes of the box at most
+template <typename R, int NT, int NB, int NP, int MODE, bool W>
+__global__ __launch_bounds__(NT) void k_sweeps(SweepArgs<R> A) {
+    extern __shared__ __align__(16) unsigned char sweep_mem[];
+    __shared__ SolverScalars S;
+    __shared__ double red[2][16];
+    constexpr int LS = NB == 1 ? 1 : NB + 1;  // LDS stride of a position
+    R *x = (R *)sweep_mem;
+    const MG &m = A.m;
+    const BoxGeo &B = A.b;
+    const int kp = m.kp, plane = B.BJ * kp, BI = B.BI;
+    const int tid = threadIdx.x, nt = blockDim.x;
+    const int per = (B.nti * B.ntj + 7) >> 3;  // XCD x owns a contiguous range of tiles
+    const int tile = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+    if (tile >= B.nti * B.ntj) return;
+    const int ti = tile / B.ntj, tj = tile - ti * B.ntj;
+    const int ib = ti * B.TI - B.hi + 1, jb = tj * B.TJ - B.hj + 1;  // (first column, 1-based)
+    // (an axis with a halo has more than 4 columns: at most two periods off)
+    auto wrap2 = [](int i, int n) {
+        i = i < 1 ? i + n : i;
+        i = i > n ? i - n : i;
+        return i > n ? i - n : i;
+    };
+    const Coef<R> C(A.cp.m64, A.cp.m32);
+    // element e of a plane: a uniform base and a 32-bit offset per lane
+    auto at = [](const R *p, unsigned e) -> R {
+        return *(const R *)((const char *)p + e * (unsigned)sizeof(R));
+    };
+    auto put = [](R *p, unsigned e, R v) {
+        *(R *)((char *)p + e * (unsigned)sizeof(R)) = v;
+    };
+    auto at_plane = [&](int ii) { return (size_t)((wrap2(ib + ii, m.ip) - 1) * m.si); };
+    if (tid < (int)(sizeof(SolverScalars) / 8))
+        ((unsigned long long *)&S)[tid] = ((const unsigned long long *)A.in)[tid];
+    const bool fold = MODE != 2 && A.pin;
+    constexpr int NF = MODE == 0 ? 2 : 1;
+    if (fold) fold_load<NF>(A.pin, A.npin, (double *)sweep_mem);
+    // the thread's positions: plane offset in the compact vectors, LDS
+    // offsets of its own and its j and k neighbours' planes, coefficients
+    int jj[NP], q[NP], qs[NP], qn[NP], qd[NP], qu[NP];
+    unsigned g[NP];
+    R as[NP], an[NP], ad[NP], au[NP], ap[NP], y[NP];
+    const R ae = C.ae[1], aw = C.aw[1];
+    R s[NP][NB], t[NP][NB];
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+        const int pos = tid + n * nt;
+        jj[n] = -1;
+        if (pos < plane) {
+            jj[n] = (int)((unsigned)pos / (unsigned)kp);
+            const int k = pos - jj[n] * kp, j = wrap2(jb + jj[n], m.jp);
+            g[n] = (unsigned)((j - 1) * m.sj + k);
+            as[n] = C.as[j];
+            an[n] = C.an[j];
+            ad[n] = C.ad[k + 1];
+            au[n] = C.au[k + 1];
+            // (at the box's edge along j the neighbour is never used unless
+            // the axis closes on itself)
+            q[n] = pos * LS;
+            qs[n] = (pos + (jj[n] > 0 ? -kp : plane - kp)) * LS;
+            qn[n] = (pos + (jj[n] < B.BJ - 1 ? kp : kp - plane)) * LS;
+            qd[n] = (pos - (k > 0 ? 1 : 0)) * LS;
+            qu[n] = (pos + (k < kp - 1 ? 1 : 0)) * LS;
+        }
+    }
+    // the bulk of the loads, in flight while the partial sums are folded
+    // (loads return in order: what the fold needs goes first)
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+        if (jj[n] < 0) continue;
+#pragma unroll
+        for (int ii = 0; ii < NB; ++ii) {
+            if (ii >= BI) continue;
+            const size_t c = at_plane(ii);
+            s[n][ii] = at(MODE == 2 ? A.s + c : A.r + c, g[n]);
+            t[n][ii] = at(MODE == 2 ? A.t + c : A.v1 + c, g[n]);
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+        ap[n] = (((((-ae) - aw) - an[n]) - as[n]) - au[n]) - ad[n];
+        y[n] = recip(ap[n]);
+    }
+    if (MODE != 2) {
+        double f[NF];
+        if (fold) fold_sum<NF>(A.npin, (double *)sweep_mem, f);
+        __syncthreads();
+        if (tid == 0) {
+            if (fold && !(S.breakdown | S.done)) {
+                if constexpr (MODE == 0)
+                    fin_r_apply(&S, f[0], f[1]);
+                else
+                    fin_v_apply(&S, f[0]);
+            }
+            if (blockIdx.x == 0) *A.out = S;
+        }
+    }
+    __syncthreads();
+    if (S.breakdown | S.done) return;
+    const R a = MODE == 0 ? (R)S.bet : (R)S.alf, bo = (R)S.omg;
+    const bool first_it = S.iters == 0;  // v1 = p = 0 (dynamics.f90:379-380)
+    const int j0 = B.hj, j1 = B.hj + B.TJ, i0 = B.hi;
+    const int i1 = min(B.hi + B.TI, m.ip - ib + 1);  // own planes [i0, i1)
+    auto own = [&](int n) { return jj[n] >= j0 && jj[n] < j1 && jb + jj[n] <= m.jp; };
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+        if (jj[n] < 0) continue;
+        const bool o = own(n) && A.t_out;
+#pragma unroll
+        for (int ii = 0; ii < NB; ++ii) {
+            if (ii >= BI) continue;
+            if (MODE != 2) {
+                const R vq = MODE == 0 && first_it ? R(0) : t[n][ii];
+                t[n][ii] = tv<R, MODE == 1 ? 1 : 0>(s[n][ii], vq, a, bo);
+                const R s0 = div_by(t[n][ii], ap[n], y[n]);
+                s[n][ii] = W ? A.w[0] * s0 : s0;
+                if (o && ii >= i0 && ii < i1)
+                    put(A.t_out + (size_t)((ib + ii - 1) * m.si), g[n], t[n][ii]);
+            }
+            x[q[n] + ii] = s[n][ii];
+            if (ii & 1) __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    __syncthreads();
+    // sweep sw on the box without its sw outermost columns
+    auto to_lds = [&](int d) {
+        const int di = B.hi ? d : 0, dj = B.hj ? d : 0;
+#pragma unroll
+        for (int n = 0; n < NP; ++n) {
+            if (jj[n] < dj || jj[n] >= B.BJ - dj) continue;
+#pragma unroll
+            for (int ii = 0; ii < NB; ++ii)
+                if (ii >= di && ii < BI - di) x[q[n] + ii] = s[n][ii];
+        }
+        __syncthreads();
+    };
+    for (int sw = 1; sw <= A.nsw; ++sw) {
+        const R w = A.w[sw];
+        const int di = B.hi ? sw : 0, dj = B.hj ? sw : 0;
+#pragma unroll
+        for (int n = 0; n < NP; ++n) {
+            if (jj[n] < dj || jj[n] >= B.BJ - dj) continue;
+            R west = s[n][0];  // the west value before its update
+            if (!B.hi) {       // a closed axis: the last plane
+#pragma unroll
+                for (int ii = 1; ii < NB; ++ii)
+                    if (ii == BI - 1) west = s[n][ii];
+            }
+            const R first = s[n][0];
+#pragma unroll
+            for (int ii = 0; ii < NB; ++ii) {
+                const R c = s[n][ii];
+                if (ii >= di && ii < BI - di) {
+                    const R east = ii == BI - 1 ? first : s[n][ii + 1 < NB ? ii + 1 : NB - 1];
+                    const R As = stencil<R>(aw, ae, as[n], an[n], ad[n], au[n], ap[n], west, east,
+                                            x[qs[n] + ii], x[qn[n] + ii], x[qd[n] + ii],
+                                            x[qu[n] + ii], c);
+                    const R d = div_by(t[n][ii] - As, ap[n], y[n]);
+                    s[n][ii] = c + (W ? w * d : d);
+                }
+                west = c;
+                // (all planes' LDS reads at once would need hundreds of registers)
+                if (ii & 1) __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        __syncthreads();
+        if (sw < A.nsw) to_lds(sw);
+    }
+    // p = s + bet*p (dynamics.f90:399); t is not needed any more
+    if (MODE != 1 && A.p_old && !first_it) {
+        const R bet = (R)S.bet;
+#pragma unroll
+        for (int n = 0; n < NP; ++n) {
+            if (jj[n] < 0) continue;
+#pragma unroll
+            for (int ii = 0; ii < NB; ++ii)
+                if (ii < BI) t[n][ii] = at(A.p_old + at_plane(ii), g[n]);
+        }
+#pragma unroll
+        for (int n = 0; n < NP; ++n)
+#pragma unroll
+            for (int ii = 0; ii < NB; ++ii)
+                if (ii < BI) s[n][ii] = s[n][ii] + bet * t[n][ii];
+    } else if (MODE != 1 && A.p_old) {
+#pragma unroll
+        for (int n = 0; n < NP; ++n)
+#pragma unroll
+            for (int ii = 0; ii < NB; ++ii)
+                if (ii < BI) s[n][ii] = s[n][ii] + (R)S.bet * R(0);
+    }
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+        if (jj[n] < 0 || !own(n)) continue;
+#pragma unroll
+        for (int ii = 0; ii < NB; ++ii)
+            if (ii >= i0 && ii < i1) {
+                const size_t c = (size_t)((ib + ii - 1) * m.si);
+                put(A.s_out + c, g[n], s[n][ii]);
+                // the dot's other factor (MODE 1: s, this kernel's t)
+                if (MODE != 1 && A.dot) t[n][ii] = at(A.dot + c, g[n]);
+            }
+    }
+    if (!A.dot) return;
+    to_lds(A.nsw);
+    // y = A s and its partial sums in the marching kernels' order: a column's
+    // planes in one thread, then the wave and block sums of its marching tile
+    double acc[NP][2];
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+        acc[n][0] = acc[n][1] = 0.0;
+        if (jj[n] < 0 || !own(n)) continue;
+        R west = s[n][0], first = s[n][0];
+        if (!B.hi) {
+#pragma unroll
+            for (int ii = 1; ii < NB; ++ii)
+                if (ii == BI - 1) west = s[n][ii];
+        }
+#pragma unroll
+        for (int ii = 0; ii < NB; ++ii) {
+            if (ii >= BI) continue;
+            const R c = s[n][ii];
+            if (ii >= i0 && ii < i1) {
+                const R east = ii == BI - 1 ? first : s[n][ii + 1 < NB ? ii + 1 : NB - 1];
+                const R yv = stencil<R>(aw, ae, as[n], an[n], ad[n], au[n], ap[n], west, east,
+                                        x[qs[n] + ii], x[qn[n] + ii], x[qd[n] + ii],
+                                        x[qu[n] + ii], c);
+                put(A.y_out + (size_t)((ib + ii - 1) * m.si), g[n], yv);
+                const R ac = t[n][ii];
+                if (A.two) {
+                    acc[n][0] += (double)yv * (double)yv;
+                    acc[n][1] += (double)yv * (double)ac;
+                } else {
+                    acc[n][0] += (double)ac * (double)yv;
+                }
+            }
+            west = c;
+            if (ii & 1) __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    // to the lane of the marching tile: [k tile][row, k in tile]
+    double *sums = (double *)sweep_mem;
+    const int nsum = 256 * m.nkb;
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+        if (jj[n] < 0 || !own(n)) continue;
+        const int k = q[n] / LS - jj[n] * kp, kb = k / m.kt;
+        const int e = kb * 256 + (jj[n] - j0) * m.kt + (k - kb * m.kt);
+        sums[e] = acc[n][0];
+        sums[nsum + e] = acc[n][1];
+    }
+    __syncthreads();
+    for (int wv = tid >> 6; wv < 4 * m.nkb; wv += nt >> 6) {
+        const int e = (wv & 3) * 64 + (tid & 63);  // the lane in its marching tile
+        const int k = (wv >> 2) * m.kt + e % m.kt, j = tj * B.TJ + e / m.kt + 1;
+        const bool act = k < kp && j <= m.jp;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const double v = wave_sum(act ? sums[c * nsum + wv * 64 + (tid & 63)] : 0.0);
+            if ((tid & 63) == 0) red[c][wv] = v;
+        }
+    }
+    __syncthreads();
+    if (tid < m.nkb) {
+        const int mt = tid + m.nkb * (tj + m.njb * ti);
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const double *rw = red[c] + 4 * tid;
+            A.pout[c * m.nblocks + mt] = ((rw[0] + rw[1]) + rw[2]) + rw[3];
+        }
+    }
+}
+
+// k_update with the fold of <t,t>, <t,s> in front of it: the same cells, sums
+// and order (update_body)
+template <typename R>
+__global__ __launch_bounds__(256) void k_update_fold(
+    R *__restrict__ x, const R *__restrict__ p, const R *__restrict__ cs,
+    const R *__restrict__ s, const R *__restrict__ t, const R *__restrict__ cr,
+    R *__restrict__ r, int n, int nbu, const SolverScalars *__restrict__ in, SolverScalars *out,
+    const double *__restrict__ pin, int npin, double *pout) {
+    __shared__ double red[2048];
+    __shared__ SolverScalars S;
+    if (threadIdx.x < sizeof(SolverScalars) / 8)
+        ((unsigned long long *)&S)[threadIdx.x] = ((const unsigned long long *)in)[threadIdx.x];
+    double f[2];
+    fold_load<2>(pin, npin, red);
+    fold_sum<2>(npin, red, f);
+    if (threadIdx.x == 0) {
+        if (!(S.breakdown | S.done)) fin_t_apply(&S, f[0], f[1]);
+        if (blockIdx.x == 0) *out = S;
+    }
+    __syncthreads();
+    if (S.breakdown | S.done) return;
+    update_body<R>(glob(x), glob(p), glob(cs), glob(s), glob(t), glob(cr), glob(r), n, nbu, &S,
+                   pout, (int)blockIdx.x);
+}
+
+// the state after the last update for the host: the residual's fold applied
+// (the next iteration's first kernel does it again for itself)
+__global__ __launch_bounds__(256) void k_poll_fold(const SolverScalars *in, SolverScalars *out,
+                                                   const double *pin, int npin, int *flags) {
+    __shared__ double red[2048];
+    double f[2];
+    fold_load<2>(pin, npin, red);
+    fold_sum<2>(npin, red, f);
+    if (threadIdx.x == 0) {
+        SolverScalars S = *in;
+        if (!(S.breakdown | S.done)) fin_r_apply(&S, f[0], f[1]);
+        *out = S;
+        *flags = (S.done ? 1 : 0) | (S.breakdown ? 2 : 0) | (S.nonfinite ? 4 : 0);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1661,6 +2094,190 @@ static int iteration_graph(dcm_ctx *c, const SolvePlan &P, const IterLaunch<R> &
     return DCM_OK;
 }
 
+// The box of a fused kernel whose group has `halo` stencil passes: tiles of
+// march planes x jt columns; an axis no longer than the tile needs no halo.
+static BoxGeo box_geo(const MG &m, int halo) {
+    BoxGeo b;
+    b.TI = m.ic;
+    b.TJ = m.jt;
+    b.hi = m.ip <= b.TI ? 0 : halo;
+    b.hj = m.jp <= b.TJ ? 0 : halo;
+    b.BI = b.hi ? b.TI + 2 * halo : m.ip;
+    b.BJ = b.hj ? b.TJ + 2 * halo : m.jp;
+    b.nti = m.nic;
+    b.ntj = m.njb;
+    return b;
+}
+
+// Whether a single system's iteration runs in the fused kernels, a rule on
+// its size and grid.  The grid is uniform along x (every grid the reference
+// makes is, initialisation.f90:429-446); the box fits the LDS of a workgroup
+// and the registers of its threads (one or two positions each), the folds'
+// partial sums their pass; and the tiles fit the chip's 256 CUs at a block
+// each: a second round of blocks doubles a launch whose columns are already
+// computed up to six times.  Measured at 228 tiles of 8 x 8 (150x91x70,
+// FP32, twelve divisions): four sweeps 17 us against 24 as four launches;
+// at 128 tiles of 8 x 4 (64^3, FP64) an iteration 51 us against 84.
+constexpr int kFuseTiles = 256;
+template <typename R> static bool sweeps_fit(const dcm_ctx *c, int planes) {
+    const Geo &g = c->geo;
+    if (!c->uniform_x || planes != 8) return false;
+    const long long n = (long long)g.ip * g.jp * g.kp;
+    const MG m = march_geo(g, planes);
+    const BoxGeo b = box_geo(m, kGroup);
+    const int pos = b.BJ * g.kp;
+    const int most = b.BI == 1 ? 2048 : (sizeof(R) == 8 ? 768 : 1536);
+    return (long long)b.nti * b.ntj <= kFuseTiles && m.nkb <= 4 && m.nblocks <= 1024 &&
+           update_blocks(n) <= 1024 && pos <= most && sweep_lds<R>(b, m) <= 155 * 1024;
+}
+
+template <typename R, int MODE, bool W>
+static int sweeps_launch(hipStream_t st, const SweepArgs<R> &a) {
+    const int pos = a.b.BJ * a.m.kp;
+    const size_t lds = sweep_lds<R>(a.b, a.m);
+    const dim3 grid((unsigned)((a.b.nti * a.b.ntj + 7) / 8 * 8));
+    auto go = [&](auto kern, int np) -> int {
+        // (per device and thread-safe in the runtime; cheap beside a launch)
+        if (lds > 64 * 1024)
+            DCM_HIP(hipFuncSetAttribute((const void *)kern,
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        const int nt = ((pos + np - 1) / np + 63) / 64 * 64;
+        hipLaunchKernelGGL(kern, grid, dim3(nt), lds, st, a);
+        return DCM_OK;
+    };
+    constexpr int NB = kBoxPlanes;
+    if (a.b.BI == 1)
+        return pos <= 1024 ? go(k_sweeps<R, 1024, 1, 1, MODE, W>, 1)
+                           : go(k_sweeps<R, 1024, 1, 2, MODE, W>, 2);
+    // (FP64: 768 threads have the registers for 16 planes, 1024 do not)
+    if constexpr (sizeof(R) == 8)
+        return go(k_sweeps<R, 768, NB, 1, MODE, W>, 1);
+    else
+        return pos > 1024 ? go(k_sweeps<R, 768, NB, 2, MODE, W>, 2)
+                          : go(k_sweeps<R, 1024, NB, 1, MODE, W>, 1);
+}
+
+// One preconditioner application and the product after it: groups of at most
+// kGroup stencil passes.  MODE 0: p = M(t) + bet*p into pn, v1 = A p into vn;
+// MODE 1: s into VS, cs = M(s), t = A cs.
+template <typename R> struct FusedSolve {
+    dcm_ctx *c;
+    const IterMember &M;
+    int np;                      // stride of the partial-sum buffers
+    R *p[2], *v1[2];             // alternating p and v1
+    int cur = 0;                 // the pair that holds the current p, v1
+    SolverScalars *sl() const { return c->solver; }
+    R *v(int i) const { return (R *)M.V[i]; }
+    bool cheb() const { return sizeof(R) == 4 && c->cheb_on && DCM_JAC_FIRST32 == 0; }
+
+    template <int MODE> int apply(const SolverScalars *in, SolverScalars *out, const double *pin,
+                                  int npin, double *pout) {
+        const bool w = cheb();
+        const int nS = w ? c->cheb_deg - 1 : 3;
+        // scratch: A leaves VS, VCS to its iterates, C the pair that the next
+        // A overwrites
+        R *scr[2] = {MODE == 0 ? v(VS) : p[1 - cur], MODE == 0 ? v(VCS) : v1[1 - cur]};
+        R *t = MODE == 0 ? v(VT) : v(VS);
+        const R *s_in = nullptr;
+        int done = 0, flip = 0;
+        while (done < nS) {
+            const int rem = nS - done;
+            const bool lastg = rem < kGroup;
+            const int n = lastg ? rem : (rem - 1 < kGroup ? rem - 1 : kGroup);
+            SweepArgs<R> a{};
+            a.m = M.m;
+            a.b = box_geo(M.m, n + (lastg ? 1 : 0));
+            a.cp = M.cp;
+            a.nsw = n;
+            a.in = done == 0 ? in : out;
+            a.out = out;
+            a.pin = done == 0 ? pin : nullptr;
+            a.npin = npin;
+            for (int q = 0; q <= n; ++q) a.w[q] = w ? (R)c->cheb_w[done + q] : R(1);
+            if (done == 0) {
+                a.r = v(VR);
+                a.v1 = v1[cur];
+                a.t_out = MODE == 1 || !lastg ? t : nullptr;
+            } else {
+                a.t = t;
+                a.s = s_in;
+            }
+            if (lastg) {
+                a.p_old = MODE == 0 ? p[cur] : nullptr;
+                a.s_out = MODE == 0 ? p[1 - cur] : v(VCS);
+                a.y_out = MODE == 0 ? v1[1 - cur] : v(VT);
+                a.dot = MODE == 0 ? v(VCR) : v(VS);
+                a.two = MODE;
+                a.pout = pout;
+            } else {
+                a.s_out = scr[flip];
+                s_in = scr[flip];
+                flip ^= 1;
+            }
+            if (done == 0)
+                DCM_CHECK(w ? (sweeps_launch<R, MODE, sizeof(R) == 4>(c->stream, a))
+                            : (sweeps_launch<R, MODE, false>(c->stream, a)));
+            else
+                DCM_CHECK(w ? (sweeps_launch<R, 2, sizeof(R) == 4>(c->stream, a))
+                            : (sweeps_launch<R, 2, false>(c->stream, a)));
+            done += n;
+        }
+        return DCM_OK;
+    }
+    // slots: 0 the state at the start and for the host, 2 after the residual,
+    // 3 after <cr,v1>, 4 after <t,t>, <t,s>
+    int iteration(bool first) {
+        double *pv = M.part, *pt = M.part + 2 * np, *pu = M.part + 4 * np;
+        const int nt = M.m.nblocks;
+        DCM_CHECK(apply<0>(first ? sl() : sl() + 4, sl() + 2, first ? nullptr : pu, M.nbu, pv));
+        cur = 1 - cur;  // p and v1 of this iteration
+        DCM_CHECK(apply<1>(sl() + 2, sl() + 3, pv, nt, pt));
+        hipLaunchKernelGGL(k_update_fold<R>, dim3(M.nbu), dim3(kBlock), 0, c->stream, v(VX),
+                           (const R *)p[cur], (const R *)v(VCS), (const R *)v(VS),
+                           (const R *)v(VT), (const R *)v(VCR), v(VR), M.n, M.nbu,
+                           (const SolverScalars *)(sl() + 3), sl() + 4, (const double *)pt, nt,
+                           pu);
+        return DCM_OK;
+    }
+    int poll(int *hflag, hipEvent_t ev) {
+        hipLaunchKernelGGL(k_poll_fold, dim3(1), dim3(256), 0, c->stream,
+                           (const SolverScalars *)(sl() + 4), sl(),
+                           (const double *)(M.part + 4 * np), M.nbu, hflag);
+        DCM_LAUNCH_CHECK();
+        DCM_HIP(hipEventRecord(ev, c->stream));
+        return DCM_OK;
+    }
+    // The next chunk of iterations is queued before the flags of the one
+    // before it are read, so the device does not wait for the host; kernels
+    // queued after convergence return at once.
+    int run(int itmax) {
+        int *hf;
+        DCM_CHECK(ensure_host_flags(c, 2, &hf));
+        for (hipEvent_t &e : c->poll_event)
+            if (!e) DCM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        int launched = 0, chunk = 0;
+        auto queue = [&]() -> int {
+            const int n = itmax - launched < kPollEvery ? itmax - launched : kPollEvery;
+            for (int q = 0; q < n; ++q) DCM_CHECK(iteration(launched + q == 0));
+            launched += n;
+            return poll(hf + (chunk & 1), c->poll_event[chunk & 1]);
+        };
+        DCM_CHECK(queue());
+        for (;;) {
+            const bool more = launched < itmax;
+            if (more) {
+                ++chunk;
+                DCM_CHECK(queue());
+                DCM_HIP(hipEventSynchronize(c->poll_event[(chunk - 1) & 1]));
+                if (((volatile int *)hf)[(chunk - 1) & 1] & 3) break;
+            } else {
+                break;
+            }
+        }
+        return DCM_OK;
+    }
+};
+
 // BiCGSTAB iterations (dynamics.f90:390-430) of a batch of independent
 // systems in lockstep, every launch serving all of them; a member that has
 // converged or broken down skips its blocks.  Each member's initial state and
@@ -1670,6 +2287,17 @@ static int iteration_graph(dcm_ctx *c, const SolvePlan &P, const IterLaunch<R> &
 template <typename R>
 static int bicgstab_iterate_batch(dcm_ctx *c, const SolveSys *sys, int nsys, int itmax,
                                   SolverOut *outs, int *status) {
+    if (itmax < 1) itmax = 1;
+    // a small single system: groups of passes per launch (the same bits)
+    const bool fused = nsys == 1 && sys[0].c == c && !c->seq_sums && !c->profiling &&
+                       !(c->mg_on && c->mg) && sweeps_fit<R>(c, sys[0].march_planes);
+    int np = 0;
+    if (fused) {
+        const int nt = march_geo(c->geo, sys[0].march_planes).nblocks;
+        const int nu = update_blocks((long long)c->geo.ip * c->geo.jp * c->geo.kp);
+        np = nt > nu ? nt : nu;
+        DCM_CHECK(ensure_partials(c, 6 * (size_t)np + 64));
+    }
     SolvePlan P;
     DCM_CHECK(plan_solve(c->stream, sys, nsys, P, c->solve_tables));
     const IterArgs &A = P.args;
@@ -1677,8 +2305,12 @@ static int bicgstab_iterate_batch(dcm_ctx *c, const SolveSys *sys, int nsys, int
     int *dflags, *hflags;
     DCM_CHECK(c->flags.ensure(sizeof(int) * nsys, (void **)&dflags));
     DCM_CHECK(ensure_host_flags(c, nsys, &hflags));
-    if (itmax < 1) itmax = 1;
     int launched = 0;
+    if (fused) {
+        FusedSolve<R> F{c, P.mem[0], np, {L.v(VP), L.v(VWA)}, {L.v(VV1), L.v(VWB)}};
+        DCM_CHECK(F.run(itmax));
+        launched = itmax;
+    }
     // A multigrid iteration is about sixty launches, most of them small
     // coarse-level kernels that finish faster than the host can queue them:
     // it is captured once as a graph and replayed (not while kernels are
