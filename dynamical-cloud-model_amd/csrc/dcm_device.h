@@ -21,6 +21,23 @@ __device__ __forceinline__ int zclamp(int k, int kp) {
     return k < 1 ? 1 : (k > kp ? kp : k);
 }
 
+// x / b by Markstein's theorem (IBM J. Res. Dev. 34, 1990): with y = 1/b
+// correctly rounded, one residual step makes x*y faithful and a second one
+// is the correctly rounded quotient, the IEEE one, in 5 operations instead
+// of a division's dozen.  The theorem needs exact residuals: quotients near
+// the ends of the exponent range take the division.
+__device__ __forceinline__ double div_by(double x, double b, double y) {
+    const double q0 = x * y;
+    const double q1 = __builtin_fma(__builtin_fma(-b, q0, x), y, q0);
+    const double q2 = __builtin_fma(__builtin_fma(-b, q1, x), y, q1);
+    const double ax = fabs(x);
+    if (__builtin_expect(!((ax >= 0x1p-900 && ax <= 0x1p900) || x == 0.0), 0)) return x / b;
+    return q2;
+}
+__device__ __forceinline__ float div_by(float x, float, float y) { return x * y; }
+__device__ __forceinline__ double recip(double b) { return 1.0 / b; }
+__device__ __forceinline__ float recip(float b) { return __builtin_amdgcn_rcpf(b); }
+
 // Linear thread / block ids for 3-D launches.
 __device__ __forceinline__ int lin_tid() {
     return threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z);
@@ -62,6 +79,41 @@ __device__ __forceinline__ double wave_sum(double v) {
     v += lane_down<4>(v);
     v += lane_down<2>(v);
     return v + lane_down<1>(v);
+}
+
+// the next (previous) lane's value; lane 63 (0) keeps its own
+__device__ __forceinline__ double next_lane(double v) {
+    union {
+        double d;
+        int u[2];
+    } x;
+    x.d = v;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+        x.u[h] = __builtin_amdgcn_update_dpp(x.u[h], x.u[h], 0x130, 0xf, 0xf, false);
+    return x.d;
+}
+__device__ __forceinline__ double prev_lane(double v) {
+    union {
+        double d;
+        int u[2];
+    } x;
+    x.d = v;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+        x.u[h] = __builtin_amdgcn_update_dpp(x.u[h], x.u[h], 0x138, 0xf, 0xf, false);
+    return x.d;
+}
+// lane l's value in every lane (l uniform)
+__device__ __forceinline__ double lane_at(double v, int l) {
+    union {
+        double d;
+        int u[2];
+    } x;
+    x.d = v;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) x.u[h] = __builtin_amdgcn_readlane(x.u[h], l);
+    return x.d;
 }
 
 // Sum NS values over a block of kBlock threads in a fixed order and store

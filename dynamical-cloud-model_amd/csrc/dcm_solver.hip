@@ -1051,23 +1051,6 @@ __global__ __launch_bounds__(256) void k_update_b(IterArgs A) {
 // between two buffers, because a block reads its neighbours' old values.
 // ---------------------------------------------------------------------------
 
-// x / b by Markstein's theorem (IBM J. Res. Dev. 34, 1990): with y = 1/b
-// correctly rounded, one residual step makes x*y faithful and a second one
-// is the correctly rounded quotient, the IEEE one, in 5 operations instead
-// of a division's dozen.  The theorem needs exact residuals: quotients near
-// the ends of the exponent range take the division.
-__device__ __forceinline__ double div_by(double x, double b, double y) {
-    const double q0 = x * y;
-    const double q1 = __builtin_fma(__builtin_fma(-b, q0, x), y, q0);
-    const double q2 = __builtin_fma(__builtin_fma(-b, q1, x), y, q1);
-    const double ax = fabs(x);
-    if (__builtin_expect(!((ax >= 0x1p-900 && ax <= 0x1p900) || x == 0.0), 0)) return x / b;
-    return q2;
-}
-__device__ __forceinline__ float div_by(float x, float, float y) { return x * y; }
-__device__ __forceinline__ double recip(double b) { return 1.0 / b; }
-__device__ __forceinline__ float recip(float b) { return __builtin_amdgcn_rcpf(b); }
-
 // reduce_slot_1024 of NS <= 2 slots of n <= 1024 values each (slot s at
 // p + s*n) by a block of any whole number of waves: the sums in every
 // thread.  red: 2048 doubles of LDS.  Split in two, so that a kernel issues

@@ -157,3 +157,46 @@ def test_full_size_sedimentation_loses_the_floor_flux():
     m1 = float((interior(got) * wgt).sum())
     assert abs((m1 - m0) - loss) <= 1e-11 * m0, (m1 - m0, loss)
     assert interior(got).min() >= 0.0
+
+
+# one to four levels a lane and their edges; the last shape takes the
+# per-pass kernels
+@pytest.mark.parametrize("shape", [(3, 2, 64), (2, 5, 65), (4, 3, 127), (3, 3, 128), (2, 3, 129),
+                                   (3, 2, 192), (2, 2, 200), (1, 3, 256), (2, 1, 257)])
+@pytest.mark.parametrize("kord,monotone,neumann", [(1, False, 2), (2, True, 0), (3, True, 1)])
+@pytest.mark.parametrize("variant", [H.MPDATA_LINKED, H.MPDATA_SFVT])
+def test_mpdata_vec_vert_columns_bitwise(shape, kord, monotone, neumann, variant):
+    dom = small_domain(*shape, stretched=True, varying_theta=True)
+    g = O.Grid(dom)
+    w = _w(dom, 31)
+    psi = np.stack([field(dom, 32 + n, -0.5 * n, 1.0 + n) for n in range(3)])
+    lbc, ubc = [0.1, -0.2, 0.3], [0.05, 0.0, 0.4]
+    O.set_mpdata_variant(variant)
+    try:
+        with H.Context(dom) as c:
+            c.set_mpdata_variant(variant)
+            dw, dpsi = c.array(w), c.array(psi)
+            ex, lb, ub = c.mpdata_vec_vert3d(0.9, dw, dpsi, 3, lbc, ubc, kord, monotone, neumann)
+            r, olb, oub = O.mpdata_vec_vert3d(g, 0.9, w, psi, lbc, ubc, kord, monotone, neumann)
+            assert ex == r == 0
+            np.testing.assert_array_equal(lb, olb)
+            np.testing.assert_array_equal(ub, oub)
+            np.testing.assert_array_equal(dpsi.get(), psi)
+    finally:
+        O.set_mpdata_variant(H.MPDATA_LINKED)
+
+
+@pytest.mark.parametrize("step,exits", [(0.0, 1), (1e-63, 1), (3e-61, 0), (2e-60, 0)])
+def test_vertical_zero_sum_decision(step, exits):
+    """The exit is decided by sum(psi - m) < 1e-60: by the largest term where
+    that is enough, by the sum where every term is below 1e-60."""
+    dom = small_domain(4, 3, 70)
+    g = O.Grid(dom)
+    psi = np.zeros(dom.shape)
+    psi[2, 1:3, 5:8] = step
+    w = _w(dom, 33)
+    with H.Context(dom) as c:
+        dw, dpsi = c.array(w), c.array(psi)
+        ex, _, _ = c.mpdata_vec_vert3d(1.0, dw, dpsi, 1, [0.0], [0.0], 1, False, 0)
+        r, _, _ = O.mpdata_vec_vert3d(g, 1.0, w, psi[None], [0.0], [0.0], 1, False, 0)
+        assert ex == r == exits
