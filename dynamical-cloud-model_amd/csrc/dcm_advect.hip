@@ -164,26 +164,19 @@ __global__ void k_to_float3(const double *u, const double *v, const double *w, f
 template <typename R>
 __global__ __launch_bounds__(256) void k_upwind_first(
     const double *psi, const double *mptr, const R *u, const R *v, const R *w, R *out, Geo g,
-    MetPack mp, R dt, int neumann, int do_sum, double *partials) {
+    MetPack mp, R dt, int neumann) {
     const M1<R> M(mp);
     const int k = blockIdx.x * blockDim.x + threadIdx.x + 1;
     const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
     const int i = blockIdx.z + 1;
-    const bool act = k <= g.kp && j <= g.jp;
+    if (k > g.kp || j > g.jp) return;
     const double m = *mptr;
-    double s[1] = {0.0};
-    if (act) {
-        const long long c = pidx(g, k, j, i);
-        auto P = [&](long long q) { return (R)(psi[q] - m); };
-        const R pc = P(c);
-        if (do_sum) s[0] = psi[c] - m;
-        R res = donor<R>(dt, u[c], u[c - g.si], v[c], v[c - g.sj], w[c], w[c - 1], pc,
-                         P(c + g.si), P(c - g.si), P(c + g.sj), P(c - g.sj), P(c + 1), P(c - 1),
-                         M.dxn[i], M.dyn[j], M.dzn[k], M.ra[k], M.ra[k - 1], M.rn[k], k, g.kp,
-                         neumann);
-        out[c] = res;
-    }
-    if (do_sum) block_sum_store<1>(s, partials, 0);
+    const long long c = pidx(g, k, j, i);
+    auto P = [&](long long q) { return (R)(psi[q] - m); };
+    out[c] = donor<R>(dt, u[c], u[c - g.si], v[c], v[c - g.sj], w[c], w[c - 1], P(c),
+                      P(c + g.si), P(c - g.si), P(c + g.sj), P(c - g.sj), P(c + 1), P(c - 1),
+                      M.dxn[i], M.dyn[j], M.dzn[k], M.ra[k], M.ra[k - 1], M.rn[k], k, g.kp,
+                      neumann);
 }
 
 // ---------------------------------------------------------------------------
@@ -530,6 +523,9 @@ __global__ void k_store_shifted(const R *src, double *psi, const double *mptr, c
     psi[c] = (double)src[c] + *mptr;
 }
 
+static int shifts_dev(dcm_ctx *c, const double *psi, int nf, const double *lbc,
+                      const double *ubc, int interior_min, double *dm, int *flag);
+
 // Shared body of mpdata_3d and mpdata_vec_3d.  u,v,w are the advecting
 // velocities in precision R (for R=float, FP32 shadows).  psi: nf fields of
 // ntot FP64 each.  lbc/ubc are host values (unshifted); the shifts m[n] and
@@ -551,36 +547,26 @@ int mpdata_core(dcm_ctx *c, R dt, const R *u, const R *v, const R *w, double *ps
     // unweighted antidiffusive velocities in the vector one (interior_min)
     const bool pd = c->mpdata_variant == 1;
     const bool weighted = !(pd && interior_min);
-    const unsigned nbmin = 1024;
-    const unsigned nbint = L.grid.x * L.grid.y * L.grid.z;
-    DCM_CHECK(ensure_partials(c, (size_t)nbint + nbmin + 16));
-    // K1: shifts (mpdata_3d :275-280, mpdata_vec_3d :1306-1312)
-    for (int n = 0; n < nf; ++n) {
-        const double *f = psi + (size_t)n * g.ntot;
-        int tok = prof_begin(c, "mpdata_min");
-        hipLaunchKernelGGL(k_min, dim3(nbmin), dim3(kBlock), 0, c->stream, f, g, interior_min,
-                           c->partials);
-        DCM_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_min_finish, dim3(1), dim3(1024), 0, c->stream, c->partials,
-                           (int)nbmin, lbc[n], ubc[n], dm + n, flag);
-        DCM_LAUNCH_CHECK();
-        prof_end(c, tok);
-    }
-    // K2: first donor pass of every field with (u,v,w); zero-sum test on field 1
+    // FP64: the marching kernels where the grid allows them
+    const bool fast = sizeof(R) == 8 && weighted && !pd && mpdata64_fast(c);
+    // K1: shifts (mpdata_3d :275-280, mpdata_vec_3d :1306-1312) and the
+    // zero-sum test on field 1 (:282-289)
+    DCM_CHECK(shifts_dev(c, psi, nf, lbc, ubc, interior_min, dm, flag));
+    // K2: first donor pass of every field with (u,v,w)
     std::vector<R *> s1(nf), s2(nf);
     for (int n = 0; n < nf; ++n) DCM_CHECK(get_buf<R>(c, kSlotPsi + n, &s1[n]));
     for (int n = 0; n < nf; ++n) {
+        const double *f = psi + (size_t)n * g.ntot;
+        if constexpr (sizeof(R) == 8)
+            if (fast) {
+                DCM_CHECK(mpdata64_donor1(c, dt, f, dm + n, u, v, w, s1[n], neumann));
+                continue;
+            }
         int tok = prof_begin(c, "upwind_first");
-        hipLaunchKernelGGL(k_upwind_first<R>, L.grid, L.block, 0, c->stream,
-                           psi + (size_t)n * g.ntot, dm + n, u, v, w, s1[n], g, mp, dt, neumann,
-                           n == 0 ? 1 : 0, c->partials);
+        hipLaunchKernelGGL(k_upwind_first<R>, L.grid, L.block, 0, c->stream, f, dm + n, u, v, w,
+                           s1[n], g, mp, dt, neumann);
         DCM_LAUNCH_CHECK();
         prof_end(c, tok);
-        if (n == 0) {
-            hipLaunchKernelGGL(k_exit_flag, dim3(1), dim3(1024), 0, c->stream, c->partials,
-                               (int)nbint, flag);
-            DCM_LAUNCH_CHECK();
-        }
     }
     if (kord <= 1) {
         for (int n = 0; n < nf; ++n) {
@@ -618,8 +604,14 @@ int mpdata_core(dcm_ctx *c, R dt, const R *u, const R *v, const R *w, double *ps
         for (int it = 2; it <= kord; ++it) {
             const bool last = it == kord;
             // antidiffusive velocities from the current advecting velocity
-            int tok = prof_begin(c, "antidiff");
-            if (weighted)
+            int tok = -1;
+            if constexpr (sizeof(R) == 8)
+                if (fast)
+                    DCM_CHECK(mpdata64_antidiff(c, dt, in[0], in[1], in[2], cur[0], anti[0],
+                                                anti[1], anti[2], flag));
+            if (!fast) tok = prof_begin(c, "antidiff");
+            if (fast) {
+            } else if (weighted)
                 hipLaunchKernelGGL((k_antidiff<R, true>), L.grid, L.block, 0, c->stream, in[0],
                                    in[1], in[2], cur[0], anti[0], anti[1], anti[2], flag, g, mp,
                                    dt);
@@ -632,8 +624,13 @@ int mpdata_core(dcm_ctx *c, R dt, const R *u, const R *v, const R *w, double *ps
             DCM_CHECK(fill_set<R>(c, FillSet<R>{{anti[0], anti[1], anti[2]}}, 3, FILL_FULL, 0.0,
                                   0.0, flag));
             if (monotone) {
-                tok = prof_begin(c, "beta");
-                if (pd)
+                if constexpr (sizeof(R) == 8)
+                    if (fast)
+                        DCM_CHECK(mpdata64_beta(c, dt, psi, dm, cur[0], anti[0], anti[1], anti[2],
+                                                bt.up[0], bt.dn[0], flag));
+                tok = fast ? -1 : prof_begin(c, "beta");
+                if (fast) {
+                } else if (pd)
                     hipLaunchKernelGGL((k_beta<R, true>), L.grid, L.block, 0, c->stream, psi, dm,
                                        cur[0], anti[0], anti[1], anti[2], bt, flag, g, mp, dt);
                 else
@@ -646,6 +643,14 @@ int mpdata_core(dcm_ctx *c, R dt, const R *u, const R *v, const R *w, double *ps
             }
             if (last) {
                 for (int n = 0; n < nf; ++n) {
+                    if constexpr (sizeof(R) == 8)
+                        if (fast && monotone) {
+                            DCM_CHECK(mpdata64_limited(c, dt, cur[n], anti[0], anti[1], anti[2],
+                                                       bt.up[0], bt.dn[0],
+                                                       psi + (size_t)n * g.ntot, dm + n, flag,
+                                                       neumann));
+                            continue;
+                        }
                     tok = prof_begin(c, monotone ? "upwind_limited" : "upwind_last");
                     if (monotone)
                         hipLaunchKernelGGL((k_upwind_limited<R, true>), L.grid, L.block, 0,

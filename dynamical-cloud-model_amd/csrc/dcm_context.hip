@@ -368,8 +368,13 @@ int dcm_context_create(int ip, int jp, int kp, const double *dx, const double *d
         aw[i] = 1.0 / (dx[i - 1] * dxn[i - 1]);
     }
     c->uniform_x = true;
-    for (int i = 2; i <= ip; ++i)
-        c->uniform_x = c->uniform_x && ae[i] == ae[1] && aw[i] == aw[1];
+    for (int i = 1; i <= ip + 1; ++i)
+        c->uniform_x = c->uniform_x && dx[i] == dx[0] && dxn[i] == dxn[0];
+    c->metrics_moderate = true;
+    for (const std::vector<double> *a : {&c->h_dx, &c->h_dy, &c->h_dz, &c->h_dxn, &c->h_dyn,
+                                         &c->h_dzn, &c->h_rhoa, &c->h_rhoan})
+        for (double x : *a)
+            c->metrics_moderate = c->metrics_moderate && x >= 0x1p-40 && x <= 0x1p40;
     for (int j = 1; j <= jp; ++j) {
         an[j] = 1.0 / (dy[j - 1] * dyn[j]);
         as[j] = 1.0 / (dy[j - 1] * dyn[j - 1]);

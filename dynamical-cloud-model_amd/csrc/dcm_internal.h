@@ -179,7 +179,8 @@ struct dcm_ctx {
     // scratch of the batched FP32 MPDATA: mp32_count padded FP32 fields
     float *mp32 = nullptr;
     size_t mp32_count = 0;
-    bool uniform_x = false;          // the x coefficients are the same in every plane
+    bool uniform_x = false;          // the x metrics are the same in every plane
+    bool metrics_moderate = false;   // spacings and densities within 2^-40..2^40
     std::vector<double> h_dx, h_dy, h_dz, h_dxn, h_dyn, h_dzn, h_rhoa, h_rhoan;
     // reduction scratch
     double *partials = nullptr;      // per-block partial sums (several slots)
@@ -395,6 +396,20 @@ bool mpdata32_fast(const dcm_ctx *c, int kord);
 int mpdata32_batch(dcm_ctx *c, float dt, const double *u, const double *v, const double *w,
                    float *shadow, const Mp32Cat *cats, int ncat, int kord, int monotone,
                    int neumann);
+// the FP64 passes as marching kernels (dcm_mpdata64.hip), the bits of the
+// per-cell kernels; mpdata64_fast: the grid allows them (uniform along x,
+// metrics well inside the exponent range, 32-bit byte offsets)
+bool mpdata64_fast(const dcm_ctx *c);
+int mpdata64_donor1(dcm_ctx *c, double dt, const double *psi, const double *m, const double *u,
+                    const double *v, const double *w, double *out, int neumann);
+int mpdata64_antidiff(dcm_ctx *c, double dt, const double *u, const double *v, const double *w,
+                      const double *po, double *us, double *vs, double *ws, const int *flag);
+int mpdata64_beta(dcm_ctx *c, double dt, const double *psi, const double *m, const double *po,
+                  const double *us, const double *vs, const double *ws, double *bup, double *bdn,
+                  const int *flag);
+int mpdata64_limited(dcm_ctx *c, double dt, const double *src, const double *us, const double *vs,
+                     const double *ws, const double *bup, const double *bdn, double *psi,
+                     const double *m, const int *flag, int neumann);
 // vertical-only MPDATA of nf fields (FP64); interior_min: the vector form
 int mpdata_vert_core(dcm_ctx *c, double dt, const double *w, double *psi, int nf,
                      const double *lbc, const double *ubc, int kord, int monotone, int neumann,
