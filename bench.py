@@ -16,8 +16,8 @@ W warm-up steps, then K timed steps from the same state:
 * FP64  -- the reference arithmetic (parity path);
 * mixed -- FP32 MPDATA intermediates and FP32 inner BiCGSTAB inside FP64
   iterative refinement, every solve ending at FP64 true residual < 1e-10;
-  the inner solve is preconditioned by one multigrid V-cycle per
-  application (dcm_set_precond_multigrid).  The same mixed path with the
+  the inner solve is preconditioned as dcm_set_precond_multigrid does on
+  this uniform grid, by the operator's inverse through fast transforms.  The same mixed path with the
   Chebyshev-relaxed and with the reference's plain Jacobi sweeps is
   reported beside it (paths.mixed_chebyshev, paths.mixed_plain_jacobi).
 
@@ -25,15 +25,14 @@ W warm-up steps, then K timed steps from the same state:
 wall seconds).  The ``roofline`` object describes the kernel with the
 largest time per step of that path, chosen among its candidates (the three
 FP32 MPDATA passes, each serving all ten fields in one launch, and the
-multigrid's finest-level sweep), each timed with HIP events on the model's
+preconditioner's five transform passes), each timed with HIP events on the model's
 stream in two further steps after the timed ones.  Its algorithmic bytes
 are the canonical stage bytes of the stages the kernel performs (the last
 MPDATA kernel performs two stages, the limiter and the last donor pass, so
 fusion can put its canonical figure above what it moves; ``traffic`` is what
 it moves, from the committed rocprofv3 counters).
 
-Further legs: the FP64 path with the same V-cycle (precision gain at an
-equal preconditioner), the Kelvin-Helmholtz shear layer (512x4x256, mixed
+Further legs: the FP64 path with the multigrid V-cycle of the same setting, the Kelvin-Helmholtz shear layer (512x4x256, mixed
 against FP64 error), the large domain (512x512x256, HBM footprint), the
 64-member ensemble, and the options of sources, vertical MPDATA, the
 sfvt/advection_3d.F90 arithmetic, initialisation and output.  The CPU
@@ -63,12 +62,20 @@ MPDATA32 = (("k32_donor1", "k32_donor1 (first donor pass, every field)", 24),
             ("k32_antidiff", "k32_antidiff (antidiffusive velocities, every field)", 28),
             ("k32_betalim", "k32_betalim (limiter factors + limited donor pass, every field)",
              64))
-# the headline mixed path preconditions its FP32 inner solve with a multigrid
-# V-cycle whose finest-level sweeps are the same k_jac<float,false,true>
-# (weight 0.8), five of them per inner iteration ("jac"; the sixth updates p)
-MG_DOMINANT = DOMINANT
-MG_SWEEPS_PER_ITER = 5
-MG_WORDS_PER_ITER = 51.7 # FP32 words per cell of one inner iteration (canonical)
+# the headline mixed path preconditions its FP32 inner solve with the
+# operator's inverse by transforms, applied twice per inner iteration: the five
+# passes of an application (timer "spectral") read or write 12 words per cell
+MG_DOMINANT = "spectral"
+MG_APPLICATIONS_PER_ITER = 2
+MG_APPLICATION_WORDS = 12
+# words per cell of one inner iteration (canonical): FP32 with the transforms
+# (two applications, two matvec-dots, the update), FP64 with the V-cycle (two
+# preparations of 4 words, the first sweep included, two V-cycles of three
+# sweeps of 3 words, the restriction's 2 reads and the prolongation's read and
+# write on the finest level, 13 words, 8/7 of that over all levels, two
+# matvec-dots (6), the update (8))
+SP_WORDS_PER_ITER = 38
+MG_WORDS_PER_ITER = 51.7
 PROFILE_STEPS = 2        # steps whose dominant-kernel launches are timed
 # the mixed inner solve's preconditioner: Chebyshev factors on [CHEB_A, 2]
 # with CHEB_DIVISIONS divisions by a_p (the library's default, set explicitly)
@@ -101,11 +108,7 @@ def canonical_bytes_mixed(F, inner_iters, outer, divisions=4, multigrid=False,
     # 37 FP32 words per inner iteration with the reference's four divisions,
     # each further division one more sweep (3 words) in both applications
     if multigrid:
-        # two preparations (4 words each, the first sweep included), two
-        # V-cycles (three sweeps of 3 words, the restriction's 2 reads and the
-        # prolongation's read and write on the finest level: 13 words, 8/7
-        # of that over all levels), two matvec-dots (6), the update (8)
-        b += 4 * MG_WORDS_PER_ITER * inner_iters
+        b += 4 * SP_WORDS_PER_ITER * inner_iters
     else:
         b += 4 * (37 + 6 * (divisions - 4)) * inner_iters
     b += 24 + 36                         # adv_ref_state, FP32 velocity shadows
@@ -118,7 +121,7 @@ def canonical_bytes_mixed(F, inner_iters, outer, divisions=4, multigrid=False,
 
 def run_path(H, case, precision, warmup, steps, inner_rtol=None, precond="chebyshev",
              candidates=()):
-    """precond: "multigrid" (one V-cycle per application), "chebyshev"
+    """precond: "multigrid" (dcm_set_precond_multigrid), "chebyshev"
     (Chebyshev-relaxed Jacobi sweeps) or "plain" (the reference's four
     Jacobi sweeps).  The profiled steps time the finest-level sweep and
     every kernel named in ``candidates``."""
@@ -130,7 +133,8 @@ def run_path(H, case, precision, warmup, steps, inner_rtol=None, precond="chebys
         ctx.set_precond_chebyshev(CHEB_A, CHEB_DIVISIONS)
     if precond == "multigrid":
         ctx.set_precond_multigrid(True)
-        profile_only = MG_DOMINANT
+        if precision == H.MIXED:
+            profile_only = MG_DOMINANT
     model = H.Model(ctx, case, precision)
     model.set_check_residual(True)
     if inner_rtol:
@@ -231,7 +235,7 @@ def run_ensemble(H, W, warmup, steps, members=64, seed=404, profile=False):
             x.close()
     if not profile:
         # the same ensemble with every member on the multigrid preconditioner:
-        # graphs around the solve, each member's V-cycle-preconditioned solve
+        # graphs around the solve, each member's preconditioned solve
         ctxs = [H.Context(c.dom) for c in cases]
         models = []
         try:
@@ -723,7 +727,7 @@ def kelvin_helmholtz(H, W, steps, warmup=2):
 
 def large_domain(H, W, steps, warmup=1):
     """The 512x512x256 domain (3x3 bubbles, theta + qv + 4 tracers, 25 m,
-    dt=0.25 s) on both paths, each with the V-cycle: cell-steps/s, the
+    dt=0.25 s) on both paths, each with dcm_set_precond_multigrid: cell-steps/s, the
     device memory the model holds (free memory before creation minus after
     its first step), and the canonical stage bytes per cell-step times the
     rate."""
@@ -908,7 +912,7 @@ def main(argv=None):
               f"ms/step, {res['iters_per_step']:.1f} it/step", file=sys.stderr, flush=True)
 
     if "mixed" in out and "fp64" in out and not args.no_fp64_multigrid:
-        # the FP64 path with the same V-cycle: the gain of the precision alone
+        # the FP64 path with the same setting, in FP64 the V-cycle
         print(f"[bench] FP64 with the V-cycle: warmup {args.warmup}, timed {args.steps} steps",
               file=sys.stderr, flush=True)
         res, snap, handles = run_path(H, case, H.FP64, args.warmup, args.steps,
@@ -959,13 +963,15 @@ def main(argv=None):
         # avg_launch_ms (every launch) is the figure that rocprofv3's kernel
         # statistics report.
         total_ms = k["avg_ms"] * k["launches"]
-        per_iter = MG_SWEEPS_PER_ITER if main_path == "mixed" else jac_per_iter(4)
+        mixed = main_path == "mixed"
+        per_iter = MG_APPLICATIONS_PER_ITER if mixed else jac_per_iter(4)
         active = min(k["launches"], per_iter * k["profiled_iters"])
-        cands[DOMINANT] = {
-            "kernel": ("k_jac<float,false,true> (a damped-Jacobi sweep of the V-cycle's "
-                       "finest level)" if word == 4 else "k_jac<double,false,false>"),
+        cands[MG_DOMINANT if mixed else DOMINANT] = {
+            "kernel": ("k_sp_z_fwd, k_sp_y, k_sp_x, k_sp_y, k_sp_z_inv (one application of "
+                       "the preconditioner)" if mixed else "k_jac<double,false,false>"),
             "ms_per_step": total_ms / PROFILE_STEPS,
-            "algorithmic_bytes_per_launch": JAC_WORDS * word * cells,
+            "algorithmic_bytes_per_launch": (MG_APPLICATION_WORDS if mixed else JAC_WORDS) *
+            word * cells,
             "avg_active_launch_ms": total_ms / active,
             "avg_launch_ms": k["avg_ms"], "launches": k["launches"]}
     if main_path == "mixed":

@@ -216,6 +216,8 @@ struct dcm_ctx {
     // (dcm_set_precond_multigrid; dcm_mg.hip): the hierarchy and the switch
     void *mg = nullptr;
     bool mg_on = false;
+    // its place taken in the FP32 inner solve (dcm_spectral.hip), or null
+    void *sp = nullptr;
     // levels of at most 16384 cells in one single-block kernel (default), or
     // each pass of them in its own launch (the same arithmetic)
     bool mg_tail = true;
@@ -302,6 +304,12 @@ int mg_prepare(dcm_ctx *c);
 template <typename R> int mg_correct(dcm_ctx *c, const R *b, R *x, const SolverScalars *sc);
 constexpr float kMgOmega = 0.8f;  // damped-Jacobi weight of the V-cycle's smoother
 void mg_release(dcm_ctx *c);
+// the pressure operator's inverse by fast transforms on uniform grids
+// (dcm_spectral.hip); sp_prepare leaves c->sp null where it does not apply
+int sp_prepare(dcm_ctx *c);
+void sp_release(dcm_ctx *c);
+int sp_apply(dcm_ctx *c, int mode, const float *r, const float *v1, float *t_out, float *v,
+             float *out, const SolverScalars *sc);
 
 // ---------------------------------------------------------------------------
 // resident model fields, for the output writer (dcm_dynamics.hip)

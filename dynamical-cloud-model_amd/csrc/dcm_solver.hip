@@ -1985,21 +1985,29 @@ struct IterLaunch {
         jac_launch<false, true>("jac", VWA, ti, VWB, w);
         jac_launch<P, true>(P ? "jac_p" : "jac", VWB, ti, oi, w);
     }
-    // dynamics.f90:391-425 with one V-cycle in place of each application of
-    // the Jacobi sweeps: p = V(t) + bet*p, cs = V(s)
-    void iteration_mg() const {
-        {
-            vcycle_start<0>(VT);             // t = r - bet*(omg*v1), two sweeps
-            vcycle_rest<true>(VT, VP);       // p = V(t) + bet*p
-            matvec<false>(VP, VCR, VV1);     // v1 = A p, <cr,v1>
-            fin(0);
-            vcycle_start<1>(VS);             // s = r - alf*v1, two sweeps
-            vcycle_rest<false>(VS, VCS);     // cs = V(s)
-            matvec_t_mg();                   // t = A cs, <t,t>, <t,s>
-            fin(1);
-            update_mg();                     // x, r (t recomputed); <r,r>, <r,cr>
-            fin(2, true);
+    // one application of the preconditioner: the V-cycle, or in FP32 on a
+    // uniform grid the transforms (t itself is needed only inside them)
+    template <int MODE> void precond_mg(int ti, int oi) const {
+        if constexpr (sizeof(R) == 4) {
+            if (c->sp) {
+                (void)sp_apply(c, MODE, v(VR), v(VV1), v(ti), v(VWA), v(oi), M().sc);
+                return;
+            }
         }
+        vcycle_start<MODE>(ti);
+        vcycle_rest<MODE == 0>(ti, oi);
+    }
+    // dynamics.f90:391-425 with one application of M in place of each of the
+    // Jacobi sweeps: p = M t + bet*p, cs = M s
+    void iteration_mg() const {
+        precond_mg<0>(VT, VP);       // t = r - bet*(omg*v1), p = M t + bet*p
+        matvec<false>(VP, VCR, VV1);  // v1 = A p, <cr,v1>
+        fin(0);
+        precond_mg<1>(VS, VCS);      // s = r - alf*v1, cs = M s
+        matvec_t_mg();               // t = A cs, <t,t>, <t,s>
+        fin(1);
+        update_mg();                 // x, r (t recomputed); <r,r>, <r,cr>
+        fin(2, true);
     }
     // dynamics.f90:391-425
     void iteration() const {

@@ -411,7 +411,9 @@ class Context:
 
     def set_precond_multigrid(self, on=True):
         """One multigrid V-cycle in place of the Jacobi sweeps (single models,
-        dcm_bicgstab_mixed, and the FP64 BiCGSTAB).  on=2: the same cycle
+        dcm_bicgstab_mixed, and the FP64 BiCGSTAB; the operator's inverse by
+        transforms in the mixed solve on uniform grids that halve along every
+        axis).  on=2: the same cycle
         with every pass of the coarse levels in its own launch (the default,
         True or 1, runs the levels that fit one workgroup's LDS as one
         single-block kernel; the bits are the same)."""

@@ -122,8 +122,11 @@ int dcm_fill_along_z(dcm_ctx *ctx, double *a, double lbc, double ubc);
  * Jacobi sweeps (precondition, dynamics.f90:241-270, inside :390-430), so
  * that a solve needs a few iterations at any size.  The mixed path's FP32
  * inner solve runs an FP32 V-cycle (its outer FP64 refinement still ends
- * every solve at the requested true residual); the FP64 BiCGSTAB runs the
- * same cycle in FP64, which is no longer the reference's arithmetic but
+ * every solve at the requested true residual), or, on a grid of constant
+ * spacings whose axes have only the factors 2, 3, 5 and 7 and halve together
+ * on every level, applies the operator's inverse itself by Hartley and cosine
+ * transforms in the V-cycle's place; the FP64 BiCGSTAB runs the V-cycle in
+ * FP64, which is no longer the reference's arithmetic but
  * measures the precision gain at an equal preconditioner.  DCM_BAD_ARG (and
  * no change) when the grid has at most 1024 cells or its dimensions are all
  * odd above 1024 cells.  Off by default.  In a DCM_MIXED ensemble either
@@ -136,8 +139,8 @@ int dcm_fill_along_z(dcm_ctx *ctx, double *a, double lbc, double ubc);
  * V-cycle, the levels of at most 2^17 cells as one kernel per leg and the
  * finest-level transfers as marching kernels; on = 2 launches each pass on
  * its own, one thread per cell (the same arithmetic and bits; kept for
- * comparison).  No counterpart in the
- * reference. */
+ * comparison).  The transforms are the same kernels for both.  No
+ * counterpart in the reference. */
 int dcm_set_precond_multigrid(dcm_ctx *ctx, int on);
 #define DCM_MPDATA_LINKED 0
 #define DCM_MPDATA_SFVT 1
