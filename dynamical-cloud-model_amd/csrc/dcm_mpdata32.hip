@@ -29,8 +29,8 @@
 //     column segment load them;
 //   * each pass writes, besides a cell, the halo cells that the reference's
 //     exchange would copy from it: no fill kernel runs;
-//   * the limiter factors never reach HBM: the last kernel computes them one
-//     i plane ahead into a ring of four planes in LDS (the tile's rows plus
+//   * the limiter factors never reach HBM: the last kernel computes them two
+//     i planes ahead into a ring of four planes in LDS (the tile's rows plus
 //     one halo row on each side) and applies the limited donor pass to the
 //     plane behind, so beta and the last donor pass cost one read of their
 //     inputs and one write of psi;
@@ -174,8 +174,35 @@ __device__ __forceinline__ float *beta_of(const Mp32Args &A, int L, int d) {
 template <typename T> __device__ __forceinline__ T pos0(T x) { return x > T(0) ? x : T(0); }
 template <typename T> __device__ __forceinline__ T neg0(T x) { return x < T(0) ? x : T(0); }
 __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
+// Minima and maxima as single instructions.  fminf and fmaxf of a loaded value
+// cost a second one that would quieten a signalling NaN (101 of the limiter
+// kernel's instructions); no arithmetic makes one, and of a number and a
+// quiet NaN the instruction, like fminf, gives the number.
 __device__ __forceinline__ float min3f(float a, float b, float c) {
-    return fminf(fminf(a, b), c);
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ float max3f(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+// min(1, a, b)
+__device__ __forceinline__ float unit_min(float a, float b) {
+    float r;
+    asm("v_min3_f32 %0, %1, %2, 1.0" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float pos1(float x) {
+    float r;
+    asm("v_max_f32 %0, 0, %1" : "=v"(r) : "v"(x));
+    return r;
+}
+__device__ __forceinline__ float neg1(float x) {
+    float r;
+    asm("v_min_f32 %0, 0, %1" : "=v"(r) : "v"(x));
+    return r;
 }
 __device__ __forceinline__ int wrapi(int x, int n) { return x < 1 ? x + n : (x > n ? x - n : x); }
 
@@ -686,20 +713,21 @@ __device__ __forceinline__ void beta_cell(const BetaIn &x, float rnk, float cx, 
                                           float czp, float czm, float dt, float &bu,
                                           float &bd) {
     const float small = FLT_MIN;
-    float mx = fmaxf(fmaxf(x.qc, x.qw), fmaxf(x.qe, x.qn));
-    mx = fmaxf(fmaxf(mx, x.qs), fmaxf(x.qu, x.qd));
-    mx = fmaxf(fmaxf(mx, x.oc), fmaxf(x.ow, x.oe));
-    mx = fmaxf(fmaxf(mx, x.on), fmaxf(x.os, fmaxf(x.ou, x.od)));
-    float mn = fminf(fminf(x.qc, x.qw), fminf(x.qe, x.qn));
-    mn = fminf(fminf(mn, x.qs), fminf(x.qu, x.qd));
-    mn = fminf(fminf(mn, x.oc), fminf(x.ow, x.oe));
-    mn = fminf(fminf(mn, x.on), fminf(x.os, fminf(x.ou, x.od)));
-    const float d1 = dt * ((cx * (pos0(x.uw) * x.ow - neg0(x.uc) * x.oe) +
-                            cy * (pos0(x.vl) * x.os - neg0(x.vc) * x.on)) +
-                           (czm * pos0(x.wl) * x.od - czp * neg0(x.wc) * x.ou)) +
+    float mx = max3f(max3f(x.qc, x.qw, x.qe), max3f(x.qn, x.qs, x.qu), x.qd);
+    mx = max3f(max3f(mx, x.oc, x.ow), max3f(x.oe, x.on, x.os), x.ou);
+    mx = fmaxf(mx, x.od);
+    float mn = min3f(min3f(x.qc, x.qw, x.qe), min3f(x.qn, x.qs, x.qu), x.qd);
+    mn = min3f(min3f(mn, x.oc, x.ow), min3f(x.oe, x.on, x.os), x.ou);
+    mn = fminf(mn, x.od);
+    const float uwp = pos1(x.uw), uwn = neg1(x.uw), ucp = pos1(x.uc), ucn = neg1(x.uc);
+    const float vlp = pos1(x.vl), vln = neg1(x.vl), vcp = pos1(x.vc), vcn = neg1(x.vc);
+    const float wlp = pos1(x.wl), wln = neg1(x.wl), wcp = pos1(x.wc), wcn = neg1(x.wc);
+    const float d1 = dt * ((cx * (uwp * x.ow - ucn * x.oe) +
+                            cy * (vlp * x.os - vcn * x.on)) +
+                           (czm * wlp * x.od - czp * wcn * x.ou)) +
                      small;
-    const float d2 = dt * (x.oc * ((cx * (pos0(x.uc) - neg0(x.uw)) + cy * (pos0(x.vc) - neg0(x.vl))) +
-                                   (czp * pos0(x.wc) - czm * neg0(x.wl))) +
+    const float d2 = dt * (x.oc * ((cx * (ucp - uwn) + cy * (vcp - vln)) +
+                                   (czp * wcp - czm * wln)) +
                            small);
     bu = (rnk * (mx - x.oc)) * rcp(d1);
     bd = (rnk * (x.oc - mn)) * rcp(d2);
@@ -746,7 +774,7 @@ __device__ __forceinline__ void beta_load_full(BetaIn &x, const BetaSrc &S, unsi
 // factors of the cell below the face (_c) and above it (_o)
 __device__ __forceinline__ float limited(float x, float bd_c, float bu_c, float bu_o,
                                          float bd_o) {
-    return min3f(1.f, bd_c, bu_o) * pos0(x) + min3f(1.f, bu_c, bd_o) * neg0(x);
+    return unit_min(bd_c, bu_o) * pos1(x) + unit_min(bu_c, bd_o) * neg1(x);
 }
 
 // ---------------------------------------------------------------------------
@@ -755,17 +783,24 @@ __device__ __forceinline__ float limited(float x, float bd_c, float bu_c, float 
 // the unshift, i.e. z planes (bc - m) + m.
 //
 // A block owns whole columns of kp <= 256 levels (thread t: level
-// t mod KT + 1, row t / KT of R rows) and marches a chunk of i planes.  In the
-// step for plane i it computes beta of plane i+1 -- its own rows, and the row
-// below and above the tile (the first and last rows' threads compute those
-// too; a lateral halo row takes the periodic copy's values, as
-// exchange_along_dim leaves them) -- into an LDS ring of four planes, waits
-// for the block, then applies the limited donor pass to plane i, reading the
-// factors of planes i-1, i, i+1 from the ring.  The inputs of beta for plane
-// i+1 stay in registers for the donor pass of the next step.  Four planes in
-// the ring make one barrier per step enough: the plane written in a step was
-// last read two steps earlier.  The kernel reads psi_store, never psi, which
-// it writes.
+// t mod KT + 1, row t / KT of R rows) and marches a chunk of i planes.  In
+// step i it loads the inputs of beta of plane i+1 -- its own rows, and the row
+// below and above the tile (the first and last rows' threads take those too;
+// a lateral halo row takes the periodic copy's values, as exchange_along_dim
+// leaves them) -- applies the limited donor pass to plane i-1 while those
+// loads are under way, reading the factors of planes i-2, i-1, i from an LDS
+// ring, computes beta of plane i+1 into the ring and waits for the block.  The
+// inputs of a plane's beta stay in registers for its donor pass.  Four planes
+// in the ring make one barrier per step enough: the plane written in a step
+// was last read in the step before.  The kernel reads psi_store, never psi,
+// which it writes.
+// Bound by instructions (some 230 per cell, the vector units busy 55 % of the
+// time, the rest waiting at the plane barrier for the two rows that compute
+// beta twice); tiles of 4 or 8 rows take the same time.  Measured with ten
+// fields at 256x256x128 / 512x512x256 with five: loads at the head of beta
+// and pairs of factors apart 1118 / 4557 us, loads a donor pass ahead 1042 /
+// 4351, minima and maxima as single instructions 1012 / 4163, the two factors
+// of a cell as one LDS word 979 / 4048.
 // ---------------------------------------------------------------------------
 struct K4 {
     int KT, R, njb, ntiles;  // levels per column slot, rows, tiles
@@ -780,8 +815,8 @@ static K4 k4_geo(const PM &m, int rows) {
 }
 
 __global__ __launch_bounds__(kK4Threads) void k32_betalim(Mp32Args A, PM m, K4 G, Tab32 T) {
-    // LDS ring: [plane & 3][bu, bd][row slot 0..R+1][level 0..KT-1]
-    extern __shared__ float ring[];
+    // LDS ring: [plane & 3][row slot 0..R+1][level 0..KT-1] of (bu, bd)
+    extern __shared__ float2 ring[];
     int t;
     if (!xcd_item(A.nf * G.ntiles, t)) return;
     const int f = t / G.ntiles;
@@ -798,10 +833,9 @@ __global__ __launch_bounds__(kK4Threads) void k32_betalim(Mp32Args A, PM m, K4 G
     const int i0 = icb * m.ic + 1;
     const int i1 = min(i0 + m.ic - 1, m.ip);
     const bool act = r < G.R && k <= m.kp && j <= jlast;
-    const int KT = G.KT, RS = G.R + 2, PL = 2 * RS * KT;
-    auto slot = [&](int p, int a, int rs, int kk) -> float & {
-        return ring[(p & 3) * PL + a * RS * KT + rs * KT + kk];
-    };
+    const int KT = G.KT, PL = (G.R + 2) * KT;
+    // the thread's level of a row slot
+    auto slot = [&](int p, int rs) { return ring + (p & 3) * PL + rs * KT + (k - 1); };
     const float *sto = store_of(A, L);
     const float *lp1 = psi1_of(A, lf);
     const float *us = ustar_of(A, L, 0), *vs = ustar_of(A, L, 1), *ws = ustar_of(A, L, 2);
@@ -820,89 +854,97 @@ __global__ __launch_bounds__(kK4Threads) void k32_betalim(Mp32Args A, PM m, K4 G
     const float czl = ((dt * T.ra[kk - 1]) * T.idzn[kk]) * T.irn[kk];
     const double zb = (A.lbc[f] - mm) + mm, zt = (A.ubc[f] - mm) + mm;
     const int nm = A.neumann;
-    // the halo rows this thread also computes: the row below the tile (first
-    // row) and above it (last row), as periodic copies
+    // the halo row this thread also computes: the row below the tile (first
+    // row) or above it (last row), as periodic copies; the thread of a tile
+    // of one row computes both
     const bool below = act && j == j0;
     const bool above = act && j == jlast;
-    const int jbelow = wrapi(j0 - 1, m.jp), jabove = wrapi(jlast + 1, m.jp);
+    const int jabove = wrapi(jlast + 1, m.jp);
     const int rs_above = jlast - j0 + 2;
+    const int jh = below ? wrapi(j0 - 1, m.jp) : jabove;
+    const int rsh = below ? 0 : rs_above;
+    const float cy = rnk * T.idyn[jj], cyh = rnk * T.idyn[below || above ? jh : 1];
     const BetaSrc S(sto, lp1, us, vs, ws, SI4, SJ4);
-    // beta at plane p, row jr, every input loaded
-    auto beta_at = [&](int p, int jr, BetaIn &x, float &bu, float &bd) {
-        const int pp = wrapi(p, m.ip);
-        const unsigned o = (unsigned)(pp * SI4 + jr * SJ4 + k + kK0) * 4u;
-        beta_load_full(x, S, o);
-        beta_cell(x, rnk, rnk * T.xpk[pp].y, rnk * T.idyn[jr], czp, czm, dt, bu, bd);
+    auto offset = [&](int p, int jr) {
+        return (unsigned)(wrapi(p, m.ip) * SI4 + jr * SJ4 + k + kK0) * 4u;
     };
-    auto halo_rows = [&](int p) {
-        BetaIn x;
+    // beta at plane p of loaded inputs, into row slot rs of the ring
+    auto beta_put = [&](int p, int rs, const BetaIn &x, float cyr) {
         float bu, bd;
-        if (below) {
-            beta_at(p, jbelow, x, bu, bd);
-            slot(p, 0, 0, k - 1) = bu;
-            slot(p, 1, 0, k - 1) = bd;
-        }
-        if (above) {
-            beta_at(p, jabove, x, bu, bd);
-            slot(p, 0, rs_above, k - 1) = bu;
-            slot(p, 1, rs_above, k - 1) = bd;
+        beta_cell(x, rnk, rnk * T.xpk[wrapi(p, m.ip)].y, cyr, czp, czm, dt, bu, bd);
+        *slot(p, rs) = make_float2(bu, bd);
+    };
+    auto above_too = [&](int p) {
+        BetaIn x;
+        beta_load_full(x, S, offset(p, jabove));
+        beta_put(p, rs_above, x, rnk * T.idyn[jabove]);
+    };
+    // what the donor pass reads of a plane
+    struct Don {
+        float oc, ow, oe, on, os, ou, od, uc, vc, vl, wc, wl;
+        __device__ __forceinline__ void take(const BetaIn &x) {
+            oc = x.oc, ow = x.ow, oe = x.oe, on = x.on, os = x.os, ou = x.ou, od = x.od;
+            uc = x.uc, vc = x.vc, vl = x.vl, wc = x.wc, wl = x.wl;
         }
     };
-    BetaIn cur, nxt;
+    Don cur, nxt;  // planes i-1 and i
+    float qc = 0.f, uw0 = 0.f;
     // prologue: beta of planes i0-1 (the centre of plane i0-1 is all the
     // donor pass reads of it) and i0
     if (act) {
-        float bu, bd;
-        beta_at(i0 - 1, j, cur, bu, bd);
-        slot(i0 - 1, 0, r + 1, k - 1) = bu;
-        slot(i0 - 1, 1, r + 1, k - 1) = bd;
-        beta_at(i0, j, cur, bu, bd);
-        slot(i0, 0, r + 1, k - 1) = bu;
-        slot(i0, 1, r + 1, k - 1) = bd;
-        halo_rows(i0);
+        BetaIn x, h;
+        beta_load_full(x, S, offset(i0 - 1, j));
+        beta_put(i0 - 1, r + 1, x, cy);
+        beta_load_full(x, S, offset(i0, j));
+        if (below || above) beta_load_full(h, S, offset(i0, jh));
+        beta_put(i0, r + 1, x, cy);
+        if (below || above) beta_put(i0, rsh, h, cyh);
+        if (below && above) above_too(i0);
+        nxt.take(x);
+        qc = x.qc;
+        uw0 = x.uw;
     }
     const bool jedge = j == 1 || j == m.jp;
     int c8 = i0 * SI + j * SJ + k;
     int c4 = i0 * SI4 + j * SJ4 + k + kK0;
     unsigned o4n = (unsigned)(c4 + SI4) * 4u;  // plane i+1 of the own column
     float fxl = 0.f;
-    for (int i = i0; i <= i1; ++i) {
-        // beta of plane i+1
-        if (act) {
-            float bu, bd;
-            if (i + 1 <= m.ip) {
-                // the plane before i+1 is cur's: its centre values are the
+    // step i: the loads of plane i+1, the donor pass of plane i-1 while they
+    // are under way, beta of plane i+1
+    for (int i = i0; i <= i1 + 1; ++i) {
+        BetaIn x, h;
+        const bool more = act && i <= i1;
+        if (more) {
+            if (i < m.ip) {
+                // the plane before i+1 is nxt's: its centre values are the
                 // west values of plane i+1
-                beta_load(nxt, S, o4n);
-                nxt.qw = cur.qc;
-                nxt.ow = cur.oc;
-                nxt.uw = cur.uc;
-                beta_cell(nxt, rnk, rnk * T.xpk[i + 1].y, rnk * T.idyn[j], czp, czm, dt, bu, bd);
+                beta_load(x, S, o4n);
+                x.qw = qc;
+                x.ow = nxt.oc;
+                x.uw = nxt.uc;
             } else {
-                beta_at(i + 1, j, nxt, bu, bd);
+                beta_load_full(x, S, offset(i + 1, j));
             }
-            slot(i + 1, 0, r + 1, k - 1) = bu;
-            slot(i + 1, 1, r + 1, k - 1) = bd;
-            if (i < i1) halo_rows(i + 1);
+            if (i < i1 && (below || above)) beta_load_full(h, S, offset(i + 1, jh));
         }
-        __syncthreads();
-        if (act) {
-            // the donor pass of field f at plane i with the limited velocities
-            const float buc = slot(i, 0, r + 1, k - 1), bdc = slot(i, 1, r + 1, k - 1);
-            const float bue = slot(i + 1, 0, r + 1, k - 1), bde = slot(i + 1, 1, r + 1, k - 1);
-            const float bun = slot(i, 0, r + 2, k - 1), bdn = slot(i, 1, r + 2, k - 1);
-            const float bus = slot(i, 0, r, k - 1), bds = slot(i, 1, r, k - 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (act && i > i0) {
+            // the donor pass of field f at plane i-1 with the limited
+            // velocities
+            const int q = i - 1;
+            const float2 *own = slot(q, r + 1);
+            const float2 bc = *own, be = *slot(i, r + 1), bn = own[KT], bs = own[-KT];
             // the factors vanish on the z planes (lbc = ubc = 0)
-            const float buu = k < m.kp ? slot(i, 0, r + 1, k) : 0.f;
-            const float bdu = k < m.kp ? slot(i, 1, r + 1, k) : 0.f;
-            const float uc = limited(cur.uc, bdc, buc, bue, bde);
-            const float vc = limited(cur.vc, bdc, buc, bun, bdn);
-            const float vl = limited(cur.vl, bds, bus, buc, bdc);
-            const float wc = limited(cur.wc, bdc, buc, buu, bdu);
+            const float2 bt = k < m.kp ? own[1] : make_float2(0.f, 0.f);
+            const float uc = limited(cur.uc, bc.y, bc.x, be.x, be.y);
+            const float vc = limited(cur.vc, bc.y, bc.x, bn.x, bn.y);
+            const float vl = limited(cur.vl, bs.y, bs.x, bc.x, bc.y);
+            const float wc = limited(cur.wc, bc.y, bc.x, bt.x, bt.y);
             float wl = 0.f;  // the face below k = 1 is the lbc = 0 plane
-            if (k > 1)
-                wl = limited(cur.wl, slot(i, 1, r + 1, k - 2), slot(i, 0, r + 1, k - 2), buc,
-                             bdc);
+            if (k > 1) {
+                const float2 bb = own[-1];
+                wl = limited(cur.wl, bb.y, bb.x, bc.x, bc.y);
+            }
             // psi1 of field f (for the category's first field: the values
             // beta read)
             float pc = cur.oc, pw = cur.ow, pe = cur.oe, pn = cur.on, ps = cur.os, pu = cur.ou,
@@ -916,16 +958,16 @@ __global__ __launch_bounds__(kK4Threads) void k32_betalim(Mp32Args A, PM m, K4 G
                 pu = p1[c4 + 1];
                 pd = p1[c4 - 1];
             }
-            if (i == i0) {
-                const float ul = limited(cur.uw, slot(i - 1, 1, r + 1, k - 1),
-                                         slot(i - 1, 0, r + 1, k - 1), buc, bdc);
-                fxl = pos0(ul) * pw + neg0(ul) * pc;
+            if (q == i0) {
+                const float2 bw = *slot(q - 1, r + 1);
+                const float ul = limited(uw0, bw.y, bw.x, bc.x, bc.y);
+                fxl = pos1(ul) * pw + neg1(ul) * pc;
             }
-            const float fxr = pos0(uc) * pc + neg0(uc) * pe;
-            const float fyr = pos0(vc) * pc + neg0(vc) * pn;
-            const float fyl = pos0(vl) * ps + neg0(vl) * pc;
-            float fzr = (pos0(wc) * pc + neg0(wc) * pu) * czr;
-            float fzl = (pos0(wl) * pd + neg0(wl) * pc) * czl;
+            const float fxr = pos1(uc) * pc + neg1(uc) * pe;
+            const float fyr = pos1(vc) * pc + neg1(vc) * pn;
+            const float fyl = pos1(vl) * ps + neg1(vl) * pc;
+            float fzr = (pos1(wc) * pc + neg1(wc) * pu) * czr;
+            float fzl = (pos1(wl) * pd + neg1(wl) * pc) * czl;
             if (nm == 1) {
                 if (k == 1) fzl = fzr;
                 if (k == m.kp) fzr = fzl;
@@ -933,19 +975,29 @@ __global__ __launch_bounds__(kK4Threads) void k32_betalim(Mp32Args A, PM m, K4 G
                 if (k == 1) fzl = -fzr;
                 if (k == m.kp) fzr = -fzl;
             }
-            const float cx = dt * T.xpk[i].y;
+            const float cx = dt * T.xpk[q].y;
             const float res = ((pc - (fxr - fxl) * cx) - (fyr - fyl) * cyd) - (fzr - fzl);
             const double rv = (double)res + mm;
             psi[c8] = rv;
             if (k == 1) psi[c8 - 1] = zb;
             if (k == m.kp) psi[c8 + 1] = zt;
-            if (jedge || i == 1 || i == m.ip) put_images<double>(psi, c8, rv, k, j, i, m, SJ, SI);
+            if (jedge || q == 1 || q == m.ip) put_images<double>(psi, c8, rv, k, j, q, m, SJ, SI);
             fxl = fxr;
-            cur = nxt;
+            c8 += SI;
+            c4 += SI4;
         }
-        c8 += SI;
-        c4 += SI4;
-        o4n += (unsigned)SI4 * 4u;
+        if (more) {
+            beta_put(i + 1, r + 1, x, cy);
+            if (i < i1) {
+                if (below || above) beta_put(i + 1, rsh, h, cyh);
+                if (below && above) above_too(i + 1);
+            }
+            cur = nxt;
+            nxt.take(x);
+            qc = x.qc;
+            o4n += (unsigned)SI4 * 4u;
+        }
+        __syncthreads();
     }
 }
 
