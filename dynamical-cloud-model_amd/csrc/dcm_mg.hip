@@ -52,8 +52,8 @@
 // the advection kernels of the model step, which fill the CUs, a 256-thread
 // block finds a free slot sooner than a 1024-thread one (the step 5.90 ->
 // 5.84 ms, with the 2048-cell level moved to the fused legs).  A hierarchy
-// whose level of 513..2048 cells cannot run as fused legs (a
-// semi-coarsened pair) takes a 1024-thread block with that level in it.
+// whose level of 513..2048 cells cannot run as fused legs (an odd ip or kp
+// that keeps its size) takes a 1024-thread block with that level in it.
 // The kernels and the hierarchy exist in FP32 (the mixed path's inner solve)
 // and FP64 (the FP64 BiCGSTAB with the V-cycle in place of the reference's
 // sweeps, which separates the precision gain from the preconditioner gain).
@@ -73,6 +73,11 @@ constexpr int kDenseMax = 512;     // coarsest levels solved by the dense invers
                                    // (O(n^3) host work at set-up)
 constexpr int kDenseTarget = 64;   // the hierarchy halves on toward this size
 constexpr int kFuseMax = 1 << 17;  // largest level whose legs run as one kernel each
+// smallest finest level whose transfers march: an iteration at 512x4x256 (0.5 M
+// cells) 238 us marching, 224 with a thread per cell; at 176x176x64 (2.0 M)
+// equal; at 208x112x80 (1.9 M) 355 against 363
+constexpr int kMarchMin = 1 << 20;
+constexpr int kNarrow = 8;         // rows of a narrow level, whole in a leg's box
 
 template <typename R> struct Lv {
     int ip, jp, kp, n;
@@ -458,6 +463,14 @@ __global__ __launch_bounds__(kCoarseMax) void k_mg_coarse(const R *__restrict__ 
 //         less one column, x'' = t + w (b - A t)/a_p on the tile, written to
 //         a second array (other blocks still read x in their halos).
 // Threads: x along k (blockDim.x = kp), y over the box's columns.
+// Narrow (a level of at most kNarrow rows): the tile and its box are TI planes
+// of whole rows, which need no halo along j (the neighbours wrap within the
+// box: 6 x 2 columns instead of 6 x 6 at two rows), and the next level may
+// keep the rows (a semi-coarsened pair).  Measured at 512x4x256, down and up
+// leg: 256x2x128 14.1 and 13.1 -> 6.5 and 6.0 us, 128x1x64 26 us of six
+// launches -> 12, 64x1x32 out of the tail's 1024-thread block (23.4 us) into
+// legs of its own (12) before a 256-thread one (14.0); an iteration 278 ->
+// 238 us.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int wrap1(int v, int n) {
     // 1-based periodic index of v (v may lie a few cells outside 1..n)
@@ -468,6 +481,7 @@ __device__ __forceinline__ int wrap1(int v, int n) {
 
 struct Tile2 {
     int TI, TJ;  // tile size in i and j (each a divisor of the level's ip, jp)
+    bool narrow = false;
 };
 
 // The box's 1-D coefficients: ae, aw at the BI box columns' i (wrapped), an,
@@ -498,26 +512,29 @@ __device__ __forceinline__ R box_ap(const BoxCoef<R> &B, int ii, int jj) {
     return (((((-B.ae[ii]) - B.aw[ii]) - B.an[jj]) - B.as[jj]) - B.au) - B.ad;
 }
 // A v at box element e (plane = BJ*kp, row = kp): the operator of ax_of
-template <typename R>
+template <bool N, typename R>
 __device__ __forceinline__ R ax_box(const BoxCoef<R> &B, const R *v, int e, int plane, int kp,
                                     int k, int ii, int jj, R ap) {
     const int kd = k == 1 ? 0 : 1, ku = k == kp ? 0 : 1;
-    return B.aw[ii] * v[e - plane] + B.ae[ii] * v[e + plane] + B.as[jj] * v[e - kp] +
-           B.an[jj] * v[e + kp] + B.ad * v[e - kd] + B.au * v[e + ku] + ap * v[e];
+    const int js = N && jj == 0 ? plane - kp : -kp;
+    const int jn = N && (jj + 1) * kp == plane ? kp - plane : kp;
+    return B.aw[ii] * v[e - plane] + B.ae[ii] * v[e + plane] + B.as[jj] * v[e + js] +
+           B.an[jj] * v[e + jn] + B.ad * v[e - kd] + B.au * v[e + ku] + ap * v[e];
 }
 
-template <typename R>
+template <typename R, bool N>
 __global__ __launch_bounds__(256) void k_mg_down(const R *__restrict__ b, R *__restrict__ xg,
                                                  R *__restrict__ bc, Lv<R> F, Lv<R> C,
                                                  Tile2 T, R w, const SolverScalars *sc) {
     extern __shared__ __align__(16) unsigned char mg_lds[];
     if (stopped(sc)) return;
-    const int kp = F.kp, BI = T.TI + 4, BJ = T.TJ + 4;
+    const int kp = F.kp, BI = T.TI + 4, BJ = N ? F.jp : T.TJ + 4;
+    const int hj = N ? 0 : 2, ej = N ? 0 : 1;  // the halo along j, one column less
     const int plane = BJ * kp, box = BI * plane;
     R *lb = reinterpret_cast<R *>(mg_lds), *lt = lb + box, *lx = lt + box;
     const int ntj = F.jp / T.TJ;
     const int ti = (int)blockIdx.x / ntj, tj = (int)blockIdx.x - ti * ntj;
-    const int ib = ti * T.TI - 1, jb = tj * T.TJ - 1;  // global i, j of box column (0, 0)
+    const int ib = ti * T.TI - 1, jb = tj * T.TJ + 1 - hj;  // global i, j of box column (0, 0)
     const int k = (int)threadIdx.x + 1;
     const BoxCoef<R> B = box_coef(F, lx + box, ib, jb, BI, BJ, k);
     // b of the box
@@ -536,44 +553,47 @@ __global__ __launch_bounds__(256) void k_mg_down(const R *__restrict__ b, R *__r
     }
     __syncthreads();
     // x = t + w (b - A t)/a_p on the box less one column
-    for (int col = threadIdx.y; col < (BI - 2) * (BJ - 2); col += blockDim.y) {
-        const int ii = 1 + col / (BJ - 2), jj = 1 + col % (BJ - 2);
+    for (int col = threadIdx.y; col < (BI - 2) * (BJ - 2 * ej); col += blockDim.y) {
+        const int ii = 1 + col / (BJ - 2 * ej), jj = ej + col % (BJ - 2 * ej);
         const int e = (ii * BJ + jj) * kp + (k - 1);
         const R ap = box_ap(B, ii, jj);
         const R inv = inv_of<R>(ap);
-        lx[e] = lt[e] + w * (lb[e] - ax_box(B, (const R *)lt, e, plane, kp, k, ii, jj, ap)) * inv;
+        lx[e] = lt[e] + w * (lb[e] - ax_box<N>(B, (const R *)lt, e, plane, kp, k, ii, jj, ap)) * inv;
     }
     __syncthreads();
     // x on the tile
     for (int col = threadIdx.y; col < T.TI * T.TJ; col += blockDim.y) {
-        const int ii = 2 + col / T.TJ, jj = 2 + col % T.TJ;
+        const int ii = 2 + col / T.TJ, jj = hj + col % T.TJ;
         xg[at(F, k, jb + jj, ib + ii)] = lx[(ii * BJ + jj) * kp + (k - 1)];
     }
-    // the coarse cells of the tile: mean over the eight children of (b - A x)
+    // the coarse cells of the tile: mean over the eight children of (b - A x),
+    // over four where the next level keeps the rows
     // (the children's k differ from the thread's: their au, ad from F)
     if (k <= C.kp) {
-        const int K = k;
-        for (int col = threadIdx.y; col < (T.TI / 2) * (T.TJ / 2); col += blockDim.y) {
-            const int ci = col / (T.TJ / 2), cj = col % (T.TJ / 2);
-            const int I = ti * (T.TI / 2) + ci + 1, J = tj * (T.TJ / 2) + cj + 1;
+        const int K = k, nj = N && F.jp == C.jp ? 1 : 2;
+        const int CJ = T.TJ / nj;
+        for (int col = threadIdx.y; col < (T.TI / 2) * CJ; col += blockDim.y) {
+            const int ci = col / CJ, cj = col % CJ;
+            const int I = ti * (T.TI / 2) + ci + 1, J = tj * CJ + cj + 1;
             R acc = R(0);
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
+                if (N && nj == 1 && ((q >> 1) & 1)) continue;
                 const int kk = 2 * K - 1 + (q & 1);
-                const int ii = 2 * ci + 2 + ((q >> 2) & 1), jj = 2 * cj + 2 + ((q >> 1) & 1);
+                const int ii = 2 * ci + 2 + ((q >> 2) & 1), jj = nj * cj + hj + ((q >> 1) & 1);
                 const int e = (ii * BJ + jj) * kp + (kk - 1);
                 BoxCoef<R> Bq = B;
                 Bq.au = F.au[kk];
                 Bq.ad = F.ad[kk];
                 const R ap = box_ap(Bq, ii, jj);
-                acc += lb[e] - ax_box(Bq, (const R *)lx, e, plane, kp, kk, ii, jj, ap);
+                acc += lb[e] - ax_box<N>(Bq, (const R *)lx, e, plane, kp, kk, ii, jj, ap);
             }
-            bc[at(C, K, J, I)] = R(0.125) * acc;
+            bc[at(C, K, J, I)] = (nj == 1 ? R(0.25) : R(0.125)) * acc;
         }
     }
 }
 
-template <typename R>
+template <typename R, bool N>
 __global__ __launch_bounds__(256) void k_mg_up(const R *__restrict__ xc,
                                                const R *__restrict__ xg,
                                                const R *__restrict__ b, R *__restrict__ xo,
@@ -581,12 +601,13 @@ __global__ __launch_bounds__(256) void k_mg_up(const R *__restrict__ xc,
                                                const SolverScalars *sc) {
     extern __shared__ __align__(16) unsigned char mg_lds[];
     if (stopped(sc)) return;
-    const int kp = F.kp, BI = T.TI + 4, BJ = T.TJ + 4;
+    const int kp = F.kp, BI = T.TI + 4, BJ = N ? F.jp : T.TJ + 4;
+    const int hj = N ? 0 : 2, ej = N ? 0 : 1;  // the halo along j, one column less
     const int plane = BJ * kp, box = BI * plane;
     R *lb = reinterpret_cast<R *>(mg_lds), *lt = lb + box, *lx = lt + box;
     const int ntj = F.jp / T.TJ;
     const int ti = (int)blockIdx.x / ntj, tj = (int)blockIdx.x - ti * ntj;
-    const int ib = ti * T.TI - 1, jb = tj * T.TJ - 1;
+    const int ib = ti * T.TI - 1, jb = tj * T.TJ + 1 - hj;
     const int k = (int)threadIdx.x + 1;
     const BoxCoef<R> B = box_coef(F, lx + box, ib, jb, BI, BJ, k);
     // x' = x + P xc on the whole box (trilinear, as k_mg_prolong), b staged
@@ -598,39 +619,44 @@ __global__ __launch_bounds__(256) void k_mg_up(const R *__restrict__ xc,
         const int ii = col / BJ, jj = col - ii * BJ;
         const int i = wrap1(ib + ii, F.ip), j = wrap1(jb + jj, F.jp);
         const int e = col * kp + (k - 1);
-        const int I = (i + 1) >> 1, J = (j + 1) >> 1;
-        int I2 = (i & 1) ? I - 1 : I + 1;
-        int J2 = (j & 1) ? J - 1 : J + 1;
-        I2 = I2 < 1 ? C.ip : (I2 > C.ip ? 1 : I2);
-        J2 = J2 < 1 ? C.jp : (J2 > C.jp ? 1 : J2);
-        const R a = R(0.75), q = R(0.25);
-        const R v =
-            a * (a * (a * xc[at(C, K, J, I)] + q * xc[at(C, K2, J, I)]) +
-                 q * (a * xc[at(C, K, J2, I)] + q * xc[at(C, K2, J2, I)])) +
-            q * (a * (a * xc[at(C, K, J, I2)] + q * xc[at(C, K2, J, I2)]) +
-                 q * (a * xc[at(C, K, J2, I2)] + q * xc[at(C, K2, J2, I2)]));
+        R v;
+        if (N) {
+            v = prolong_semi(F, C, xc, k, j, i);
+        } else {
+            const int I = (i + 1) >> 1, J = (j + 1) >> 1;
+            int I2 = (i & 1) ? I - 1 : I + 1;
+            int J2 = (j & 1) ? J - 1 : J + 1;
+            I2 = I2 < 1 ? C.ip : (I2 > C.ip ? 1 : I2);
+            J2 = J2 < 1 ? C.jp : (J2 > C.jp ? 1 : J2);
+            const R a = R(0.75), q = R(0.25);
+            v =
+                a * (a * (a * xc[at(C, K, J, I)] + q * xc[at(C, K2, J, I)]) +
+                     q * (a * xc[at(C, K, J2, I)] + q * xc[at(C, K2, J2, I)])) +
+                q * (a * (a * xc[at(C, K, J, I2)] + q * xc[at(C, K2, J, I2)]) +
+                     q * (a * xc[at(C, K, J2, I2)] + q * xc[at(C, K2, J2, I2)]));
+        }
         const int c = at(F, k, j, i);
         lx[e] = xg[c] + v;
         lb[e] = b[c];
     }
     __syncthreads();
     // t = x' + w (b - A x')/a_p on the box less one column
-    for (int col = threadIdx.y; col < (BI - 2) * (BJ - 2); col += blockDim.y) {
-        const int ii = 1 + col / (BJ - 2), jj = 1 + col % (BJ - 2);
+    for (int col = threadIdx.y; col < (BI - 2) * (BJ - 2 * ej); col += blockDim.y) {
+        const int ii = 1 + col / (BJ - 2 * ej), jj = ej + col % (BJ - 2 * ej);
         const int e = (ii * BJ + jj) * kp + (k - 1);
         const R ap = box_ap(B, ii, jj);
         const R inv = inv_of<R>(ap);
-        lt[e] = lx[e] + w * (lb[e] - ax_box(B, (const R *)lx, e, plane, kp, k, ii, jj, ap)) * inv;
+        lt[e] = lx[e] + w * (lb[e] - ax_box<N>(B, (const R *)lx, e, plane, kp, k, ii, jj, ap)) * inv;
     }
     __syncthreads();
     // x'' = t + w (b - A t)/a_p on the tile
     for (int col = threadIdx.y; col < T.TI * T.TJ; col += blockDim.y) {
-        const int ii = 2 + col / T.TJ, jj = 2 + col % T.TJ;
+        const int ii = 2 + col / T.TJ, jj = hj + col % T.TJ;
         const int e = (ii * BJ + jj) * kp + (k - 1);
         const R ap = box_ap(B, ii, jj);
         const R inv = inv_of<R>(ap);
         xo[at(F, k, jb + jj, ib + ii)] =
-            lt[e] + w * (lb[e] - ax_box(B, (const R *)lt, e, plane, kp, k, ii, jj, ap)) * inv;
+            lt[e] + w * (lb[e] - ax_box<N>(B, (const R *)lt, e, plane, kp, k, ii, jj, ap)) * inv;
     }
 }
 
@@ -947,10 +973,20 @@ bool mg_possible(const Geo &g) {
 // coarsest level of at most one cell per thread (its solve is one cell per
 // thread); else no tail.  The block has kTailThreads threads, or
 // kTailThreadsMax when that admits a level that fused legs cannot take.
+// A narrow level's legs: two planes of whole rows per block, the planes halved
+template <typename R> static size_t narrow_lds(const Lv<R> &L) {
+    return (3 * (size_t)6 * L.jp * L.kp + 2 * (size_t)(6 + L.jp)) * sizeof(R);
+}
+template <typename R> static bool narrow_fits(const Lv<R> &L, const Lv<R> &C) {
+    return L.jp <= kNarrow && L.ip == 2 * C.ip && L.kp == 2 * C.kp &&
+           (L.jp == C.jp || L.jp == 2 * C.jp) && narrow_lds(L) <= 64 * 1024;
+}
 template <typename R> static bool fusable(const MgLevels<R> &V, int l, int nlev) {
     if (l < 1 || l >= nlev - 1) return false;
     const Lv<R> &L = V.lv[l];
-    if (L.kp > 256 || L.n > kFuseMax || !halves(L, V.lv[l + 1])) return false;
+    if (L.kp > 256 || L.n > kFuseMax) return false;
+    if (narrow_fits(L, V.lv[l + 1])) return true;
+    if (!halves(L, V.lv[l + 1])) return false;
     for (int t : {4, 2}) {
         const size_t bytes =
             (3 * (size_t)(t + 4) * (t + 4) * L.kp + 4 * (size_t)(t + 4)) * sizeof(R);
@@ -1026,6 +1062,12 @@ template <typename R> static int plan_tiles(MgLevels<R> &V, int nlev) {
         const Lv<R> &L = V.lv[l];
         V.tile[l] = Tile2{0, 0};
         if (!fusable(V, l, nlev)) continue;
+        if (narrow_fits(L, V.lv[l + 1])) {
+            V.tile[l] = Tile2{2, L.jp, true};
+            V.tile_lds[l] = narrow_lds(L);
+            most = std::max(most, V.tile_lds[l]);
+            continue;
+        }
         for (int t : {4, 2}) {
             const size_t bytes =
                 (3 * (size_t)(t + 4) * (t + 4) * L.kp + 4 * (size_t)(t + 4)) * sizeof(R);
@@ -1039,13 +1081,11 @@ template <typename R> static int plan_tiles(MgLevels<R> &V, int nlev) {
     }
     if (most > 0) {
         // the bound every tile obeys (the attribute is shared by every context)
-        if (hipFuncSetAttribute((const void *)k_mg_down<R>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                                64 * 1024) != hipSuccess ||
-            hipFuncSetAttribute((const void *)k_mg_up<R>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                                64 * 1024) != hipSuccess)
-            return DCM_HIP_ERROR;
+        for (const void *kern : {(const void *)k_mg_down<R, false>, (const void *)k_mg_down<R, true>,
+                                 (const void *)k_mg_up<R, false>, (const void *)k_mg_up<R, true>})
+            if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    64 * 1024) != hipSuccess)
+                return DCM_HIP_ERROR;
     }
     return DCM_OK;
 }
@@ -1248,9 +1288,10 @@ int mg_correct(dcm_ctx *c, const R *b0, R *x0, const SolverScalars *sc) {
             hipLaunchKernelGGL((k_mg_prolong<R, true>), GF.grid, GF.block, 0, c->stream, xc, x,
                                V.lv[l], V.lv[l + 1], sc);
     };
-    // the marching finest transfers (mode 1, a halving first level); per-pass
-    // mode keeps the one-thread-per-cell kernels
-    const bool march = c->mg_tail && halves(V.lv[0], V.lv[1]);
+    // the marching finest transfers (mode 1, a halving first level of enough
+    // cells for its columns to fill the chip); per-pass mode keeps the
+    // one-thread-per-cell kernels
+    const bool march = c->mg_tail && halves(V.lv[0], V.lv[1]) && V.lv[0].n >= kMarchMin;
     if (march) {
         Grid3 GM = grid3(V.lv[1]);
         GM.grid.z = (unsigned)((V.lv[1].ip + kProPlanes / 2 - 1) / (kProPlanes / 2));
@@ -1268,8 +1309,9 @@ int mg_correct(dcm_ctx *c, const R *b0, R *x0, const SolverScalars *sc) {
             const Tile2 T = V.tile[l];
             const dim3 blk((unsigned)F.kp, (unsigned)(256 / F.kp));
             const unsigned nb = (unsigned)((F.ip / T.TI) * (F.jp / T.TJ));
-            hipLaunchKernelGGL(k_mg_down<R>, dim3(nb), blk, V.tile_lds[l], c->stream,
-                               (const R *)V.b[l], V.x[l], V.b[l + 1], F, C, T, w, sc);
+            const auto down = T.narrow ? k_mg_down<R, true> : k_mg_down<R, false>;
+            hipLaunchKernelGGL(down, dim3(nb), blk, V.tile_lds[l], c->stream, (const R *)V.b[l],
+                               V.x[l], V.b[l + 1], F, C, T, w, sc);
             continue;
         }
         const Grid3 GF = grid3(F);
@@ -1293,7 +1335,8 @@ int mg_correct(dcm_ctx *c, const R *b0, R *x0, const SolverScalars *sc) {
             const Tile2 T = V.tile[l];
             const dim3 blk((unsigned)F.kp, (unsigned)(256 / F.kp));
             const unsigned nb = (unsigned)((F.ip / T.TI) * (F.jp / T.TJ));
-            hipLaunchKernelGGL(k_mg_up<R>, dim3(nb), blk, V.tile_lds[l], c->stream, below,
+            const auto leg = T.narrow ? k_mg_up<R, true> : k_mg_up<R, false>;
+            hipLaunchKernelGGL(leg, dim3(nb), blk, V.tile_lds[l], c->stream, below,
                                (const R *)V.x[l], (const R *)V.b[l], V.t[l], F, C, T, w, sc);
             below = V.t[l];
             continue;
