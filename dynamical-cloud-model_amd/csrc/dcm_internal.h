@@ -232,7 +232,8 @@ struct dcm_ctx {
     dcm::DeviceScratch solve_tables, flags;
     int *h_flags = nullptr;
     size_t h_flags_cap = 0;
-    // the fused small-system solve: the flags of its last two chunks are there
+    // the host copies of the state after the last two chunks are there (the
+    // fused small-system solve; the chunked mixed solve uses the first)
     hipEvent_t poll_event[2] = {nullptr, nullptr};
     // the stream is borrowed (an ensemble's), not owned
     bool borrowed_stream = false;
