@@ -8,7 +8,7 @@
 // A V-cycle with a fixed number of sweeps is a fixed linear map, as BiCGSTAB
 // requires of its preconditioner, and it reduces every frequency of the
 // error alike, so the inner solve needs a few iterations at any size.  On
-// uniform grids that halve along every axis dcm_spectral.hip takes its place
+// uniform grids that halve along every axis at once dcm_spectral.hip takes its place
 // in the FP32 inner solve.  The
 // FP64 path keeps the reference's algorithm; the outer FP64 refinement
 // decides convergence either way.
@@ -1373,9 +1373,12 @@ int dcm_set_precond_multigrid(dcm_ctx *c, int on) {
     if (!c) return DCM_BAD_ARG;
     if (on) {
         DCM_CHECK(mg_prepare(c));
-        // every level halves along every axis: see sp_prepare
-        const int halvings = (1 << (((MgHier *)c->mg)->nlev - 1)) - 1;
-        if (((c->geo.ip | c->geo.jp | c->geo.kp) & halvings) == 0) DCM_CHECK(sp_prepare(c));
+        // every level halves along every axis, and the coarsest has two cells
+        // or more along each: see sp_prepare
+        const int f = 1 << (((MgHier *)c->mg)->nlev - 1);
+        const Geo &g = c->geo;
+        if (((g.ip | g.jp | g.kp) & (f - 1)) == 0 && std::min({g.ip, g.jp, g.kp}) >= 2 * f)
+            DCM_CHECK(sp_prepare(c));
         c->mg_on = true;
         c->mg_tail = on != 2;
     } else {

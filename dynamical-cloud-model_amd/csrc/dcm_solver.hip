@@ -2692,10 +2692,10 @@ static int mixed_one_chunked(dcm_ctx *c, const SolveTask &t, double tol, int itm
 // Several single-system multigrid mixed solves at once, system q on
 // streams[q] (its context's stream while it runs): each unfinished system in
 // turn is polled and given its next chunk, so the systems' small kernels
-// overlap on the device and none waits for the slowest (twelve uneven
-// domains: the step 4.01 ms with a drain of every stream per round, 3.77
-// ms so).  Each system runs
-// exactly the kernels of its solo solve, so it ends with the same bits.
+// overlap on the device and none waits for the slowest (6 % of the step of
+// twelve uneven domains against a drain of every stream per round).  Each
+// system runs exactly the kernels of its solo solve, so it ends with the same
+// bits.
 int bicgstab_mixed_concurrent(const SolveTask *tasks, int n, const hipStream_t *streams,
                               double tol, int itmax, const double *inner_rtol, SolverOut *outs,
                               int *status) {

@@ -26,7 +26,7 @@
 // (512x512x256, beside the advection: 270 to 430 us a pass of 0.54 GB) and by
 // the passes' latency below (128x96x64: 7 to 10 us each).
 // Measured, a mixed solve to 1e-10 with the V-cycle and with this: 128x96x64
-// 1594 -> 456 us, 32x192x96 1777 -> 453, 1024x16x16 1605 -> 675; a model step
+// 1594 -> 456 us, 112x112x80 1664 -> 649, 64x160x128 1792 -> 530; a model step
 // at 256x256x128 (9 tracers) 6.00 -> 4.14 ms, at 512x512x256 34.5 -> 23.7.
 #include <cmath>
 #include <algorithm>
@@ -421,12 +421,14 @@ void sp_release(dcm_ctx *c) {
 // The transforms' tables, when the grid allows them: constant spacings along
 // every axis, line lengths of at most 1024 with factors 2, 3, 5 and 7 only
 // (a larger factor would make its stage a direct sum of as many terms).
-// The caller leaves grids whose hierarchy is semi-coarsened (a thin axis) to
-// the V-cycle, although this is faster there too (a 512x4x256 step 3.6 ms
-// against 0.6): the two agree in p up to its undetermined constant, which
-// these transforms keep and the V-cycle's rounding lets wander, on such
-// grids by up to 4e-6 of p within some steps, more than the 2e-6 to which the
-// mixed path's results are held; where every axis halves it is below 4e-7.
+// The caller leaves grids with a thin axis to the V-cycle -- a semi-coarsened
+// hierarchy, or one that ends at one cell along some axis -- although this is
+// faster there too (a 512x4x256 step 3.6 ms against 0.6): the two agree in p
+// up to its undetermined constant, which these transforms keep and the
+// V-cycle's rounding lets wander, on such grids by up to 1.2e-6 of p in a
+// solve and 4e-6 within some steps, more than the 3e-7 and 2e-6 to which the
+// mixed path's results are held.  Over 80 grids of the others it was 2e-8 at
+// the median and 3e-7 at most.
 int sp_prepare(dcm_ctx *c) {
     if (c->sp) return DCM_OK;
     const Geo &g = c->geo;

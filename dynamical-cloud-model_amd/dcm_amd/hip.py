@@ -413,8 +413,7 @@ class Context:
         """One multigrid V-cycle in place of the Jacobi sweeps (single models,
         dcm_bicgstab_mixed, and the FP64 BiCGSTAB; the operator's inverse by
         transforms in the mixed solve on uniform grids that halve along every
-        axis).  on=2: the same cycle
-        with every pass of the coarse levels in its own launch (the default,
+        axis at once).  on=2: the same cycle with every pass of the coarse levels in its own launch (the default,
         True or 1, runs the levels that fit one workgroup's LDS as one
         single-block kernel; the bits are the same)."""
         _call("dcm_set_precond_multigrid", self.h, 2 if on == 2 else int(bool(on)))

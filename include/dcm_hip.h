@@ -124,7 +124,7 @@ int dcm_fill_along_z(dcm_ctx *ctx, double *a, double lbc, double ubc);
  * inner solve runs an FP32 V-cycle (its outer FP64 refinement still ends
  * every solve at the requested true residual), or, on a grid of constant
  * spacings whose axes have only the factors 2, 3, 5 and 7 and halve together
- * on every level, applies the operator's inverse itself by Hartley and cosine
+ * on every level, to two cells or more on the coarsest, applies the operator's inverse itself by Hartley and cosine
  * transforms in the V-cycle's place; the FP64 BiCGSTAB runs the V-cycle in
  * FP64, which is no longer the reference's arithmetic but
  * measures the precision gain at an equal preconditioner.  DCM_BAD_ARG (and
