@@ -74,8 +74,8 @@ MG_APPLICATION_WORDS = 12
 # sweeps of 3 words, the restriction's 2 reads and the prolongation's read and
 # write on the finest level, 13 words, 8/7 of that over all levels, two
 # matvec-dots (6), the update (8))
-SP_WORDS_PER_ITER = 38
-MG_WORDS_PER_ITER = 51.7
+MG_WORDS_PER_ITER = 38
+VCYCLE_WORDS_PER_ITER = 51.7
 PROFILE_STEPS = 2        # steps whose dominant-kernel launches are timed
 # the mixed inner solve's preconditioner: Chebyshev factors on [CHEB_A, 2]
 # with CHEB_DIVISIONS divisions by a_p (the library's default, set explicitly)
@@ -108,7 +108,7 @@ def canonical_bytes_mixed(F, inner_iters, outer, divisions=4, multigrid=False,
     # 37 FP32 words per inner iteration with the reference's four divisions,
     # each further division one more sweep (3 words) in both applications
     if multigrid:
-        b += 4 * SP_WORDS_PER_ITER * inner_iters
+        b += 4 * MG_WORDS_PER_ITER * inner_iters
     else:
         b += 4 * (37 + 6 * (divisions - 4)) * inner_iters
     b += 24 + 36                         # adv_ref_state, FP32 velocity shadows
@@ -1015,7 +1015,7 @@ def main(argv=None):
                                         multigrid=pth == "mixed")
         elif pth == "fp64_multigrid":
             # the V-cycle's canonical words in FP64 (twice the FP32 bytes)
-            bpc = 8.0 * (39 + 27 * F) + 2 * 4 * MG_WORDS_PER_ITER * res["iters_per_step"]
+            bpc = 8.0 * (39 + 27 * F) + 2 * 4 * VCYCLE_WORDS_PER_ITER * res["iters_per_step"]
         else:
             bpc = canonical_bytes_fp64(F, res["iters_per_step"])
         step_roof[pth] = {"bytes_per_cell_step": bpc,
