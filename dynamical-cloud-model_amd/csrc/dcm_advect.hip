@@ -7,9 +7,9 @@
 //
 // Data flow of one mpdata_3d / mpdata_vec_3d call (kord=2, limiter on):
 //   K1 min        m = min(psi)  (whole array for mpdata_3d, interior and per
-//                 field for the vector variant), combined with lbc/ubc
-//   K2 upwind-1   psi1 = donor(psi-m, u,v,w) into scratch; the same kernel
-//                 sums psi-m over the interior for the zero-sum exit test
+//                 field for the vector variant), combined with lbc/ubc, and
+//                 the interior's maximum for the zero-sum exit test
+//   K2 upwind-1   psi1 = donor(psi-m, u,v,w) into scratch
 //   K3 antidiff   U*,V*,W* from (u,v,w, psi1)           Smolarkiewicz 1984
 //   K4 beta       beta_up/beta_down from psi-m, psi1, U* Smolarkiewicz &
 //                 Grabowski 1990 eqs 19-20
@@ -22,6 +22,9 @@
 // reference's order, so the FP64 path reproduces the reference bit for bit
 // (built with -ffp-contract=off).  The zero-sum exit (:284-289) is decided on
 // the device; later kernels test the flag, so no host synchronisation occurs.
+//
+// On grids uniform along x the FP64 passes K2 to K5 are the marching kernels of
+// dcm_mpdata64.hip, with the same bits.
 //
 // The same kernels instantiated with R=float give the mixed-precision path:
 // psi1, U*, beta and the velocity shadows are FP32 (half the bytes), while

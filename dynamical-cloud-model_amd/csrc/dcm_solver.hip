@@ -32,7 +32,8 @@
 // cells in registers; j and k neighbours come through L1/L2.  Offsets are
 // 32-bit and blocks are renumbered so that each XCD (block id mod 8) walks a
 // contiguous range of tiles, which keeps the j-neighbour columns in its own
-// L2.
+// L2.  A single small system runs its sweeps in groups instead, three launches
+// an iteration (k_sweeps, sweeps_fit).
 //
 // Mixed precision (dcm_bicgstab_mixed): the same kernels with FP32 vectors
 // and FP64 dot products solve A d = r for the FP64 residual r = b - A x; the

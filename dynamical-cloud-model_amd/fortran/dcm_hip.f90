@@ -239,8 +239,9 @@ module dcm_hip
             type(c_ptr), value :: ctx
             integer(c_int), value :: order
         end function
-        ! the mixed inner solve's preconditioner: one multigrid V-cycle per
-        ! application (on /= 0) instead of the Jacobi sweeps
+        ! the mixed inner solve's preconditioner (on /= 0): one multigrid
+        ! V-cycle per application, or on uniform grids the operator's inverse
+        ! by transforms, instead of the Jacobi sweeps
         integer(c_int) function dcm_set_precond_multigrid(ctx, on) &
                 bind(c, name="dcm_set_precond_multigrid")
             import :: c_int, c_ptr
