@@ -314,7 +314,8 @@ def sedimentation(H, W, calls=20, cpu=True):
             c.mpdata_vec_vert3d(0.5, dw, dpsi, nq, [0.0] * nq, [0.0] * nq, 1, False, 2)
         wall = (time.perf_counter() - t0) / calls
     canonical = 8.0 * (2 * nq + 1) * cells
-    moved = 8.0 * (6 * nq + nq) * cells
+    # each field read by the minimum and by the pass, and written; w
+    moved = 8.0 * (3 * nq + 1) * cells
     out = {"call": "mpdata_vec_vert_3d, 3 fields, kord 1, no limiter, neumann 2",
            "grid": "256x256x128", "ms_per_call": 1e3 * wall,
            "cell_steps_per_s": cells / wall,
