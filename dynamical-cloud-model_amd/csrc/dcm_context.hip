@@ -117,40 +117,35 @@ int work_field32(dcm_ctx *c, int slot, float **out) {
     return DCM_OK;
 }
 
-int ensure_partials_adv(dcm_ctx *c, size_t n) {
-    if (c->partials_adv_cap >= n) return DCM_OK;
-    DCM_CHECK(no_alloc_in_capture(c, "ensure_partials_adv"));
-    if (c->partials_adv) {
+// The captured phases of a step hold the addresses of this scratch as kernel
+// arguments: a buffer that moves counts in scratch_moves, which is part of
+// their keys, so a graph with the old address is not replayed.
+static int grow_partials(dcm_ctx *c, double **buf, size_t *cap, size_t n, const char *what) {
+    if (*cap >= n) return DCM_OK;
+    DCM_CHECK(no_alloc_in_capture(c, what));
+    if (*buf) {
         DCM_HIP(hipStreamSynchronize(c->stream));
-        DCM_HIP(hipFree(c->partials_adv));
-        c->partials_adv = nullptr;
+        DCM_HIP(hipFree(*buf));
+        *buf = nullptr;
+        *cap = 0;
+        ++c->scratch_moves;
     }
     void *p = nullptr;
     if (hipMalloc(&p, n * sizeof(double)) != hipSuccess) {
         set_error("hipMalloc of reduction partials failed");
         return DCM_OUT_OF_MEMORY;
     }
-    c->partials_adv = (double *)p;
-    c->partials_adv_cap = n;
+    *buf = (double *)p;
+    *cap = n;
     return DCM_OK;
 }
 
+int ensure_partials_adv(dcm_ctx *c, size_t n) {
+    return grow_partials(c, &c->partials_adv, &c->partials_adv_cap, n, "ensure_partials_adv");
+}
+
 int ensure_partials(dcm_ctx *c, size_t n) {
-    if (c->partials_cap >= n) return DCM_OK;
-    DCM_CHECK(no_alloc_in_capture(c, "ensure_partials"));
-    if (c->partials) {
-        DCM_HIP(hipStreamSynchronize(c->stream));
-        DCM_HIP(hipFree(c->partials));
-        c->partials = nullptr;
-    }
-    void *p = nullptr;
-    if (hipMalloc(&p, n * sizeof(double)) != hipSuccess) {
-        set_error("hipMalloc of reduction partials failed");
-        return DCM_OUT_OF_MEMORY;
-    }
-    c->partials = (double *)p;
-    c->partials_cap = n;
-    return DCM_OK;
+    return grow_partials(c, &c->partials, &c->partials_cap, n, "ensure_partials");
 }
 
 int ensure_solver_vectors64(dcm_ctx *c, size_t count) {

@@ -1341,10 +1341,12 @@ static int run_phase(hipStream_t stream, PhaseGraph *slots, const std::vector<in
 
 }  // namespace dcm
 
-// what the kernels of a captured phase and their arguments depend on
+// what the kernels of a captured phase and their arguments depend on, the
+// addresses of the context's scratch among it
 static std::vector<int> phase_key(const dcm_model *m) {
     return {m->n % 2 + 3 * (m->precision == DCM_MIXED) + 6 * (m->c->seq_sums ? 1 : 0) +
-            12 * m->c->mpdata_variant + 24 * m->gen};
+                12 * m->c->mpdata_variant + 24 * m->gen,
+            m->c->scratch_moves};
 }
 
 // Run phase 0 (before the solve) or 1 (after it) of a model step: eagerly
@@ -1751,7 +1753,7 @@ int dcm_ensemble_step(dcm_ensemble *e, int nsteps, dcm_step_stats *stats) {
     const int n = (int)e->mem.size();
     if (stats) std::memset(stats, 0, sizeof(dcm_step_stats) * n);
     std::vector<SolverOut> outs;
-    std::vector<int> key(n);
+    std::vector<int> key;
     auto pre = [&]() -> int {
         return fan_out(e, [](dcm_model *m) { return model_pre_solve(m); });
     };
@@ -1772,15 +1774,17 @@ int dcm_ensemble_step(dcm_ensemble *e, int nsteps, dcm_step_stats *stats) {
         if (v.size() >= 48) v.erase(v.begin());
         v.push_back(key);
     };
+    auto members_key = [&]() {
+        key.clear();
+        for (const dcm_model *m : e->mem) {
+            const std::vector<int> k = phase_key(m);
+            key.insert(key.end(), k.begin(), k.end());
+        }
+    };
     for (int s = 0; s < nsteps; ++s) {
         bool graphs = e->use_graphs;
-        for (int q = 0; q < n; ++q) {
-            // what the captured kernels and their arguments depend on
-            const dcm_model *m = e->mem[q];
-            key[q] = m->n % 2 + 3 * (m->precision == DCM_MIXED) + 6 * (m->c->seq_sums ? 1 : 0) +
-                     12 * m->c->mpdata_variant + 24 * m->gen;
-            graphs = graphs && !m->c->profiling;
-        }
+        for (int q = 0; q < n; ++q) graphs = graphs && !e->mem[q]->c->profiling;
+        members_key();
         if (graphs && seen(0)) {
             DCM_CHECK(run_phase(e->stream, e->pre, key, pre, [] {}));
         } else {
@@ -1798,6 +1802,7 @@ int dcm_ensemble_step(dcm_ensemble *e, int nsteps, dcm_step_stats *stats) {
             add_stats(stats ? stats + q : nullptr, outs[q], true_resid);
             if (stats) stats[q].steps += 1;
         }
+        members_key();  // the solve may have moved scratch
         if (graphs && seen(1)) {
             DCM_CHECK(run_phase(e->stream, e->post, key, post, advance_levels));
         } else {

@@ -187,6 +187,7 @@ struct dcm_ctx {
     size_t partials_cap = 0;         // doubles
     double *partials_adv = nullptr;  // the FP32 MPDATA's, which may run beside the solve
     size_t partials_adv_cap = 0;
+    int scratch_moves = 0;           // times partials, partials_adv or mp32 have moved
     double *dscal = nullptr;         // generic device scalars (64 doubles)
     double *hscal = nullptr;         // pinned host mirror (64 doubles)
     dcm::SolverScalars *solver = nullptr;   // device (5: the solve's state, and the fused kernels' slots)

@@ -1156,6 +1156,7 @@ static int ensure_mp32(dcm_ctx *c, size_t count, size_t ntot4) {
         DCM_HIP(hipFree(c->mp32));
         c->mp32 = nullptr;
         c->mp32_count = 0;
+        ++c->scratch_moves;
     }
     void *p = nullptr;
     const size_t bytes = count * ntot4 * sizeof(float);
