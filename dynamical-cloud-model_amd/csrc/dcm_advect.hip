@@ -8,7 +8,7 @@
 // Data flow of one mpdata_3d / mpdata_vec_3d call (kord=2, limiter on):
 //   K1 min        m = min(psi)  (whole array for mpdata_3d, interior and per
 //                 field for the vector variant), combined with lbc/ubc, and
-//                 the interior's maximum for the zero-sum exit test
+//                 the interior's maximum and sum for the zero-sum exit test
 //   K2 upwind-1   psi1 = donor(psi-m, u,v,w) into scratch
 //   K3 antidiff   U*,V*,W* from (u,v,w, psi1)           Smolarkiewicz 1984
 //   K4 beta       beta_up/beta_down from psi-m, psi1, U* Smolarkiewicz &
@@ -1117,13 +1117,17 @@ __global__ __launch_bounds__(256) void k_vert_columns(const double *__restrict__
 }
 
 // Per block, the minimum of field blockIdx.z over the whole array (or the
-// interior) and, of field 0, the maximum over the interior, for
-// k_minmax_finish.  A block walks planes i; a plane's rows are contiguous.
+// interior) and, of field 0 over the interior, the maximum and the sum of psi
+// - r, r its first cell, for k_minmax_finish.  A block walks planes i; a
+// plane's rows are contiguous.  partials: the minima of every field, then the
+// maxima and the sums of field 0.
 __global__ __launch_bounds__(256) void k_minmax(const double *__restrict__ psi, Geo g,
                                                 int interior_only, double *partials) {
     const double *a = psi + (size_t)blockIdx.z * g.ntot;
     const unsigned plane = (unsigned)g.si, nk = (unsigned)g.nk;
-    double mn = INFINITY, mx = -INFINITY;
+    const bool lead = blockIdx.z == 0;
+    const double r = lead ? a[pidx(g, 1, 1, 1)] : 0.0;
+    double mn = INFINITY, mx = -INFINITY, s = 0.0;
     for (int i = blockIdx.y; i < g.ni; i += gridDim.y) {
         const bool ii = i >= 1 && i <= g.ip;
         if (interior_only && !ii) continue;
@@ -1133,78 +1137,88 @@ __global__ __launch_bounds__(256) void k_minmax(const double *__restrict__ psi, 
             const unsigned j = e / nk, k = e - j * nk;
             const bool in = ii && k >= 1 && k <= (unsigned)g.kp && j >= 1 && j <= (unsigned)g.jp;
             if (in || !interior_only) mn = v < mn ? v : mn;
-            if (in) mx = v > mx ? v : mx;
+            if (in) {
+                mx = v > mx ? v : mx;
+                s += v - r;
+            }
         }
     }
-    __shared__ double red[2][4];
+    __shared__ double red[3][4];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
         const double o = __shfl_down(mn, off, 64), q = __shfl_down(mx, off, 64);
         mn = o < mn ? o : mn;
         mx = q > mx ? q : mx;
     }
+    s = wave_sum(s);
     if ((threadIdx.x & 63) == 0) {
         red[0][threadIdx.x >> 6] = mn;
         red[1][threadIdx.x >> 6] = mx;
+        red[2][threadIdx.x >> 6] = s;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
         for (int q = 1; q < 4; ++q) {
             mn = red[0][q] < mn ? red[0][q] : mn;
             mx = red[1][q] > mx ? red[1][q] : mx;
+            s += red[2][q];
         }
         const int nb = gridDim.x * gridDim.y, b = blockIdx.y * gridDim.x + blockIdx.x;
-        partials[(2 * blockIdx.z) * nb + b] = mn;
-        partials[(2 * blockIdx.z + 1) * nb + b] = mx;
+        partials[blockIdx.z * nb + b] = mn;
+        if (lead) {
+            const size_t o = (size_t)gridDim.z * nb + b;
+            partials[o] = mx;
+            partials[o + nb] = s;
+        }
     }
 }
 
 // The shifts m of every field (one block each), and the zero-sum exit from
-// field 0: sum(psi - m) < 1e-60 over the interior.  Every term is at least
-// zero and the largest is max - m, so the sum is only formed where that is
-// below 1e-60 too.
+// field 0: sum(psi - m) < 1e-60 over the interior (:284-289).  Every term is
+// at least zero and the largest is max - m, so the sum counts only where that
+// is below 1e-60 too; there it is sum(psi - r) + n (r - m) with r any of the
+// values, exactly zero for a constant field and NaN with a NaN or an infinity
+// among the values, as the sum of the terms themselves is.  (Rounding moves it
+// by at most about 1e-6 of the threshold: n 2^-52 terms of at most 1e-60.)
+// Summing in the pass over the field that every call makes costs nothing
+// measurable; one block summing a zero field of 256x256x128 took 3.2 of the
+// call's 3.3 ms (now 0.12).
 __global__ __launch_bounds__(1024) void k_minmax_finish(const double *partials, int nb,
                                                         VertBcs bc, const double *psi, Geo g,
                                                         double *dm, int *flag) {
-    const int n = blockIdx.x;
-    __shared__ double red[1024];
-    const double mn = reduce_min_1024(partials + 2 * (size_t)n * nb, nb);
+    const int n = blockIdx.x, t = threadIdx.x;
+    __shared__ double red[2][16];
+    const double mn = reduce_min_1024(partials + (size_t)n * nb, nb);
     const double m0 = bc.l[n] < mn ? bc.l[n] : mn, m = bc.u[n] < m0 ? bc.u[n] : m0;
-    if (threadIdx.x == 0) dm[n] = m;
+    if (t == 0) dm[n] = m;
     if (n != 0) return;
-    double mx = -INFINITY;
-    for (int b = threadIdx.x; b < nb; b += 1024) {
-        const double v = partials[nb + b];
+    const double *pmx = partials + (size_t)gridDim.x * nb, *ps = pmx + nb;
+    double mx = -INFINITY, s = 0.0;
+    for (int b = t; b < nb; b += 1024) {
+        const double v = pmx[b];
+        mx = v > mx ? v : mx;
+        s += ps[b];
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const double v = __shfl_down(mx, off, 64);
         mx = v > mx ? v : mx;
     }
-    red[threadIdx.x] = mx;
-    __syncthreads();
-    for (int w = 512; w > 0; w >>= 1) {
-        if (threadIdx.x < w)
-            red[threadIdx.x] = red[threadIdx.x + w] > red[threadIdx.x] ? red[threadIdx.x + w]
-                                                                       : red[threadIdx.x];
-        __syncthreads();
+    s = wave_sum(s);
+    if ((t & 63) == 0) {
+        red[0][t >> 6] = mx;
+        red[1][t >> 6] = s;
     }
-    mx = red[0];
     __syncthreads();
-    if (mx - m >= 1e-60) {
-        if (threadIdx.x == 0) *flag = 0;
-        return;
-    }
-    double s = 0.0;
-    for (int i = 1; i <= g.ip; ++i)
-        for (unsigned e = threadIdx.x; e < (unsigned)g.si; e += 1024) {
-            const unsigned j = e / (unsigned)g.nk, k = e - j * g.nk;
-            if (k >= 1 && k <= (unsigned)g.kp && j >= 1 && j <= (unsigned)g.jp)
-                s += psi[(long long)i * g.si + e] - m;
+    if (t == 0) {
+        for (int q = 1; q < 16; ++q) {
+            mx = red[0][q] > mx ? red[0][q] : mx;
+            s += red[1][q];
         }
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 512; w > 0; w >>= 1) {
-        if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
+        const double r = psi[pidx(g, 1, 1, 1)];
+        const double cells = (double)((long long)g.ip * g.jp * g.kp);
+        *flag = !(mx - m >= 1e-60) && s + cells * (r - m) < 1e-60;
     }
-    if (threadIdx.x == 0) *flag = red[0] < 1e-60 ? 1 : 0;
 }
 
 // minima of nf <= 32 fields into dm, the zero-sum flag of field 0
@@ -1216,7 +1230,7 @@ static int shifts_dev(dcm_ctx *c, const double *psi, int nf, const double *lbc,
     unsigned by = (unsigned)std::max<long long>(1, 2048 / ((long long)bx * nf));
     if (by > (unsigned)g.ni) by = (unsigned)g.ni;
     const int nb = (int)(bx * by);
-    DCM_CHECK(ensure_partials(c, 2 * (size_t)nb * nf + 16));
+    DCM_CHECK(ensure_partials(c, (size_t)nb * (nf + 2) + 16));
     VertBcs bc;
     for (int n = 0; n < 32; ++n) {
         bc.l[n] = n < nf ? lbc[n] : 0.0;

@@ -200,3 +200,56 @@ def test_vertical_zero_sum_decision(step, exits):
         ex, _, _ = c.mpdata_vec_vert3d(1.0, dw, dpsi, 1, [0.0], [0.0], 1, False, 0)
         r, _, _ = O.mpdata_vec_vert3d(g, 1.0, w, psi[None], [0.0], [0.0], 1, False, 0)
         assert ex == r == exits
+
+
+# a field whose largest value is no more than 1e-60 above the shift: zero, any
+# other constant, sums on both sides of the threshold with the first cell
+# below, at and above the others, and values that are not finite
+def _nearly_constant(dom, case):
+    psi = np.full(dom.shape, {"constant": 7.5, "infinite": np.inf}.get(case, 0.0))
+    inner = psi[1:-1, 1:-1, 1:-1]
+    if case == "first cell below":
+        inner[0, 0, 0] = 3e-61
+    elif case == "first cells above":
+        inner[0, 0, :4] = 3e-61
+    elif case == "last cells above":
+        inner[-1, -1, -4:] = 3e-61
+    elif case == "all but the first cell":
+        inner[...] = 2e-66
+        inner[0, 0, 0] = 0.0
+    elif case == "nan":
+        inner[-1, -1, -1] = np.nan
+    elif case == "nan in the first cell":
+        inner[0, 0, 0] = np.nan
+    return psi
+
+
+@pytest.mark.parametrize("vector", [False, True])
+@pytest.mark.parametrize("vertical", [False, True])
+@pytest.mark.parametrize("shape", [(1, 1, 2), (9, 33, 70), (70, 9, 257)])
+@pytest.mark.parametrize("case,exits", [
+    ("zero", 1), ("constant", 1), ("infinite", 0), ("first cell below", 1),
+    ("first cells above", None), ("last cells above", None), ("all but the first cell", 1),
+    ("nan", 0), ("nan in the first cell", 0)])
+def test_zero_sum_decision_of_nearly_constant_fields(shape, case, exits, vertical, vector):
+    if exits is None:  # four cells of 3e-61, or two
+        exits = int(shape == (1, 1, 2))
+    dom = small_domain(*shape)
+    psi = _nearly_constant(dom, case)
+    b = psi[0, 0, 0]
+    w = _w(dom, 33)
+    with H.Context(dom) as c:
+        vel = [c.zeros(), c.zeros(), c.array(w)]
+        # a second field that is not constant: the first decides
+        fields = [psi, field(dom, 34)] if vector else [psi]
+        d = c.array(np.stack(fields))
+        args = [1.0, vel[2], d] if vertical else [1.0, *vel, d]
+        if vector:
+            call = c.mpdata_vec_vert3d if vertical else c.mpdata_vec3d
+            ex, _, _ = call(*args, 2, [b, -1.0], [b, -1.0], 2, True, 0)
+        else:
+            call = c.mpdata_vert3d if vertical else c.mpdata3d
+            ex, _, _ = call(*args, b, b, 2, True, 0)
+        assert ex == exits
+        if exits and case in ("zero", "constant"):
+            np.testing.assert_array_equal(d.get()[0], psi)
