@@ -31,6 +31,7 @@
 // psi, the shift m and the output stay FP64.
 #include <algorithm>
 #include <cfloat>
+#include <type_traits>
 #include <vector>
 
 #include "dcm_device.h"
@@ -1128,21 +1129,28 @@ __global__ __launch_bounds__(256) void k_minmax(const double *__restrict__ psi, 
     const bool lead = blockIdx.z == 0;
     const double r = lead ? a[pidx(g, 1, 1, 1)] : 0.0;
     double mn = INFINITY, mx = -INFINITY, s = 0.0;
-    for (int i = blockIdx.y; i < g.ni; i += gridDim.y) {
-        const bool ii = i >= 1 && i <= g.ip;
-        if (interior_only && !ii) continue;
-        const double *b = a + (long long)i * g.si;
-        for (unsigned e = blockIdx.x * 256 + threadIdx.x; e < plane; e += gridDim.x * 256) {
-            const double v = b[e];
-            const unsigned j = e / nk, k = e - j * nk;
-            const bool in = ii && k >= 1 && k <= (unsigned)g.kp && j >= 1 && j <= (unsigned)g.jp;
-            if (in || !interior_only) mn = v < mn ? v : mn;
-            if (in) {
-                mx = v > mx ? v : mx;
-                s += v - r;
+    auto walk = [&](auto first) {
+        for (int i = blockIdx.y; i < g.ni; i += gridDim.y) {
+            const bool ii = i >= 1 && i <= g.ip;
+            if (interior_only && !ii) continue;
+            const double *b = a + (long long)i * g.si;
+            for (unsigned e = blockIdx.x * 256 + threadIdx.x; e < plane; e += gridDim.x * 256) {
+                const double v = b[e];
+                const unsigned j = e / nk, k = e - j * nk;
+                const bool in =
+                    ii && k >= 1 && k <= (unsigned)g.kp && j >= 1 && j <= (unsigned)g.jp;
+                if (in || !interior_only) mn = v < mn ? v : mn;
+                if (first && in) {
+                    mx = v > mx ? v : mx;
+                    s += v - r;
+                }
             }
         }
-    }
+    };
+    if (lead)
+        walk(std::true_type{});
+    else
+        walk(std::false_type{});
     __shared__ double red[3][4];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
@@ -1180,42 +1188,44 @@ __global__ __launch_bounds__(256) void k_minmax(const double *__restrict__ psi, 
 // values, exactly zero for a constant field and NaN with a NaN or an infinity
 // among the values, as the sum of the terms themselves is.  (Rounding moves it
 // by at most about 1e-6 of the threshold: n 2^-52 terms of at most 1e-60.)
-// Summing in the pass over the field that every call makes costs nothing
-// measurable; one block summing a zero field of 256x256x128 took 3.2 of the
-// call's 3.3 ms (now 0.12).
+// Summed in the pass over the field that every call makes, it costs nothing
+// measurable (a sedimentation call 187 us either way); one block summing a
+// zero field of 256x256x128 took 3.2 of the call's 3.3 ms (now 0.12).
 __global__ __launch_bounds__(1024) void k_minmax_finish(const double *partials, int nb,
                                                         VertBcs bc, const double *psi, Geo g,
                                                         double *dm, int *flag) {
     const int n = blockIdx.x, t = threadIdx.x;
     __shared__ double red[2][16];
+    double mx = -INFINITY, s = 0.0, r = 0.0;
+    if (n == 0) {
+        const double *pmx = partials + (size_t)gridDim.x * nb, *ps = pmx + nb;
+        r = psi[pidx(g, 1, 1, 1)];
+        for (int b = t; b < nb; b += 1024) {
+            const double v = pmx[b];
+            mx = v > mx ? v : mx;
+            s += ps[b];
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            const double v = __shfl_down(mx, off, 64);
+            mx = v > mx ? v : mx;
+        }
+        s = wave_sum(s);
+        if ((t & 63) == 0) {
+            red[0][t >> 6] = mx;
+            red[1][t >> 6] = s;
+        }
+    }
+    // (its barriers also publish red)
     const double mn = reduce_min_1024(partials + (size_t)n * nb, nb);
     const double m0 = bc.l[n] < mn ? bc.l[n] : mn, m = bc.u[n] < m0 ? bc.u[n] : m0;
     if (t == 0) dm[n] = m;
     if (n != 0) return;
-    const double *pmx = partials + (size_t)gridDim.x * nb, *ps = pmx + nb;
-    double mx = -INFINITY, s = 0.0;
-    for (int b = t; b < nb; b += 1024) {
-        const double v = pmx[b];
-        mx = v > mx ? v : mx;
-        s += ps[b];
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const double v = __shfl_down(mx, off, 64);
-        mx = v > mx ? v : mx;
-    }
-    s = wave_sum(s);
-    if ((t & 63) == 0) {
-        red[0][t >> 6] = mx;
-        red[1][t >> 6] = s;
-    }
-    __syncthreads();
     if (t == 0) {
         for (int q = 1; q < 16; ++q) {
             mx = red[0][q] > mx ? red[0][q] : mx;
             s += red[1][q];
         }
-        const double r = psi[pidx(g, 1, 1, 1)];
         const double cells = (double)((long long)g.ip * g.jp * g.kp);
         *flag = !(mx - m >= 1e-60) && s + cells * (r - m) < 1e-60;
     }
