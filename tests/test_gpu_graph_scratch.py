@@ -104,10 +104,10 @@ def test_second_mixed_model_on_the_context():
     _single(case, H.MIXED, grow)
 
 
-def test_ensemble_member_stepped_alone():
-    """Alone, the member's solve takes the route of a small single system."""
+def test_calls_on_an_ensemble_members_context():
     cases = [W.warm_bubble(1, 64, 64, steps=19, seed=3),
              W.warm_bubble(12, 10, 24, steps=19, seed=4)]
+    dom = cases[0].dom
 
     def run(graphs):
         ctxs = [H.Context(k.dom) for k in cases]
@@ -118,10 +118,14 @@ def test_ensemble_member_stepped_alone():
             with H.Ensemble(models) as e:
                 e.set_graphs(graphs)
                 e.step(7)
-                models[0].step(2)
-                g = _Guards(ctxs[0])
-                e.step(6)
-                g.check()
+                for nf in (8, 32):
+                    psi = ctxs[0].array(np.stack([field(dom, 40 + n, 0.0, 1.0)
+                                                  for n in range(nf)]))
+                    w = ctxs[0].array(0.1 * field(dom, 39))
+                    ctxs[0].mpdata_vec_vert3d(0.5, w, psi, nf)
+                    g = _Guards(ctxs[0])
+                    e.step(6)
+                    g.check()
             return [f for k, m in zip(cases, models) for f in _snapshot(k, m)]
         finally:
             for m in models:

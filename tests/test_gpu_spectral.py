@@ -44,6 +44,21 @@ def test_the_transforms_invert_the_operator(shape):
     assert rel_l2(x0 - x0.mean(), x - x.mean()) < 1e-7
 
 
+@pytest.mark.parametrize("shape", [(1024, 128, 128), (128, 768, 128), (128, 128, 1024)])
+def test_long_lines(shape):
+    """Lines of up to 1024 values: each refinement takes one iteration, or two
+    where FP32 rounding times the condition number, (2 n / pi)^2 / 2 times 6e-8
+    along a line of n = 768 or more, nears the inner tolerance.  Both solutions
+    leave a residual of 1e-10 of b, which may all lie in the smoothest mode,
+    1/sqrt(cells) of b and most of the solution: 2e-10 sqrt(cells) apart."""
+    dom = small_domain(*shape, delta=10.0)
+    it, outer, err, x = _solve(dom, 1)
+    assert err < 1e-10 and outer <= it <= 2 * outer, (it, outer, err)
+    _, _, err0, x0 = _solve(dom, 0)
+    assert err0 < 1e-10
+    assert rel_l2(x0 - x0.mean(), x - x.mean()) < 2e-10 * np.sqrt(x.size)
+
+
 def _stretched(*shape):
     dom = small_domain(*shape)
     f = 1.0 + 0.2 * np.random.default_rng(3).random((2, dom.kp + 2))
