@@ -25,7 +25,8 @@ __device__ __forceinline__ int zclamp(int k, int kp) {
 // correctly rounded, one residual step makes x*y faithful and a second one
 // is the correctly rounded quotient, the IEEE one, in 5 operations instead
 // of a division's dozen.  The theorem needs exact residuals: quotients near
-// the ends of the exponent range take the division.
+// the ends of the exponent range take the division.  (-0 over a positive b
+// gives +0, which no comparison tells from the quotient.)
 __device__ __forceinline__ double div_by(double x, double b, double y) {
     const double q0 = x * y;
     const double q1 = __builtin_fma(__builtin_fma(-b, q0, x), y, q0);

@@ -794,9 +794,10 @@ __device__ __forceinline__ float limited(float x, float bd_c, float bu_c, float 
 // in the ring make one barrier per step enough: the plane written in a step
 // was last read in the step before.  The kernel reads psi_store, never psi,
 // which it writes.
-// Bound by instructions (some 230 per cell, the vector units busy 55 % of the
-// time, the rest waiting at the plane barrier for the two rows that compute
-// beta twice); tiles of 4 or 8 rows take the same time.  Measured with ten
+// Bound by instructions and the plane barrier: 219 vector instructions a cell
+// by the counters, 0.47 ms of issue in 0.97 (the rest waiting at the barrier
+// for the two rows that compute beta twice), 2.73 GB of HBM traffic; tiles of
+// 4 or 8 rows take the same time.  Measured with ten
 // fields at 256x256x128 / 512x512x256 with five: loads at the head of beta
 // and pairs of factors apart 1118 / 4557 us, loads a donor pass ahead 1042 /
 // 4351, minima and maxima as single instructions 1012 / 4163, the two factors

@@ -1030,20 +1030,23 @@ __global__ __launch_bounds__(256) void k_update_b(IterArgs A) {
 // Small systems: the iteration in three kernels (seven with the default
 // twelve Chebyshev divisions) instead of 14 (29).
 //
-// Up to about a million cells every pass of the iteration above is bound by
-// its launch (3 to 7 us each against 1 to 3 us of memory time), so a system
-// that small runs whole groups of passes per launch.  A block owns a tile of
+// On a small system every pass of the iteration above is bound by its launch
+// (3 to 7 us each against 1 to 3 us of memory time), so it runs whole groups
+// of passes per launch (sweeps_fit: the largest are about a million cells in
+// FP32; in FP64 a three-dimensional grid of more than 64 levels does not fit
+// and keeps the passes above).  A block owns a tile of
 // 8 x jt columns (the marching tiles of those columns, every level), reads
 // its right-hand side with a halo as wide as the group has stencil passes,
 // keeps the iterate in registers and LDS and lets the valid region shrink by
 // one column a pass: the halo columns are recomputed (2 to 6 times the work,
 // which the idle CUs of a small grid have to spare) instead of exchanged.
-// Measured per FP64 step: 1x101x120 6.8 -> 2.7 ms, 64^3 7.5 -> 4.7 ms; of a
+// Measured per FP64 step: 1x101x120 6.4 -> 2.5 ms, 64^3 7.6 -> 4.9 ms; of a
 // 22 us launch at 64^3, the loads take 2 us, the folds and scalars 2, the
-// sweeps 8 (bound by FP64 issue), the sums and stores 4.  The one-block reductions go too: each kernel's blocks all fold
-// the partial sums of the kernel before it (the same tree, so the same bits)
-// and apply the scalar recurrence themselves; block 0 stores the result for
-// the next kernel in a slot that no block of this launch reads.
+// sweeps 8 (bound by FP64 issue), the sums and stores 4.  The one-block
+// reductions go too: each kernel's blocks all fold the partial sums of the
+// kernel before it (the same tree, so the same bits) and apply the scalar
+// recurrence themselves; block 0 stores the result for the next kernel in a
+// slot that no block of this launch reads.
 //   A: fold <r,r>,<r,cr>; t = r - bet*(omg*v1), sweeps, p, v1 = A p, <cr,v1>
 //   C: fold <cr,v1>; s = r - alf*v1, sweeps, cs, t = A cs, <t,t>, <t,s>
 //   U: fold <t,t>,<t,s>; x, r, <r,r>, <r,cr>
@@ -2104,8 +2107,9 @@ static BoxGeo box_geo(const MG &m, int halo) {
 // Whether a single system's iteration runs in the fused kernels, a rule on
 // its size and grid.  The grid is uniform along x (every grid the reference
 // makes is, initialisation.f90:429-446); the box fits the LDS of a workgroup
-// and the registers of its threads (one or two positions each), the folds'
-// partial sums their pass; and the tiles fit the chip's 256 CUs at a block
+// and the registers of its threads (one or two positions each: at 12 columns
+// along j 64 levels in FP64 and 128 in FP32, 192 and 256 where an axis of at
+// most four columns closes on itself), the folds' partial sums their pass; and the tiles fit the chip's 256 CUs at a block
 // each: a second round of blocks doubles a launch whose columns are already
 // computed up to six times.  Measured at 228 tiles of 8 x 8 (150x91x70,
 // FP32, twelve divisions): four sweeps 17 us against 24 as four launches;
@@ -2240,8 +2244,9 @@ template <typename R> struct FusedSolve {
         return DCM_OK;
     }
     // The next chunk of iterations is queued before the flags of the one
-    // before it are read, so the device does not wait for the host; kernels
-    // queued after convergence return at once.
+    // before it are read, so the device does not wait for the host; a kernel
+    // queued after convergence still loads its box before it returns (3 to 7
+    // us instead of 7 to 22).
     int run(int itmax) {
         int *hf;
         DCM_CHECK(ensure_host_flags(c, 2, &hf));
@@ -2693,10 +2698,10 @@ static int mixed_one_chunked(dcm_ctx *c, const SolveTask &t, double tol, int itm
 // Several single-system multigrid mixed solves at once, system q on
 // streams[q] (its context's stream while it runs): each unfinished system in
 // turn is polled and given its next chunk, so the systems' small kernels
-// overlap on the device and none waits for the slowest (6 % of the step of
-// twelve uneven domains against a drain of every stream per round).  Each
-// system runs exactly the kernels of its solo solve, so it ends with the same
-// bits.
+// overlap on the device and a finished chunk waits for at most one chunk of
+// each system before it in the round instead of for every stream to drain (6 %
+// of the step of twelve uneven domains).  Each system runs exactly the kernels
+// of its solo solve, so it ends with the same bits.
 int bicgstab_mixed_concurrent(const SolveTask *tasks, int n, const hipStream_t *streams,
                               double tol, int itmax, const double *inner_rtol, SolverOut *outs,
                               int *status) {

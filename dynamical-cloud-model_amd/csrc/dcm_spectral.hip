@@ -425,10 +425,13 @@ void sp_release(dcm_ctx *c) {
 // hierarchy, or one that ends at one cell along some axis -- although this is
 // faster there too (a 512x4x256 step 3.6 ms against 0.6): the two agree in p
 // up to its undetermined constant, which these transforms keep and the
-// V-cycle's rounding lets wander, on such grids by up to 1.2e-6 of p in a
-// solve and 4e-6 within some steps, more than the 3e-7 and 2e-6 to which the
-// mixed path's results are held.  Over 80 grids of the others it was 2e-8 at
-// the median and 3e-7 at most.
+// V-cycle's rounding lets wander, on such grids by up to 1.2e-6 of p in one
+// solve and 4e-6 within the first steps, more than the 3e-7 (a solve) and 2e-6
+// (a step) within which the choice of the preconditioner may move p.  Over 80
+// grids of the others it was 2e-8 at the median and 3e-7 at most.  (That is
+// not the mixed path's distance from the FP64 path, which FP32 advection
+// sets: at 256x256x128 p is 2e-8 off after two steps and 2.4e-6 after 27,
+// the same with either preconditioner and with the Chebyshev sweeps.)
 int sp_prepare(dcm_ctx *c) {
     if (c->sp) return DCM_OK;
     const Geo &g = c->geo;

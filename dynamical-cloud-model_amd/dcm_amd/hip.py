@@ -413,9 +413,10 @@ class Context:
         """One multigrid V-cycle in place of the Jacobi sweeps (single models,
         dcm_bicgstab_mixed, and the FP64 BiCGSTAB; the operator's inverse by
         transforms in the mixed solve on uniform grids that halve along every
-        axis at once).  on=2: the same cycle with every pass of the coarse levels in its own launch (the default,
-        True or 1, runs the levels that fit one workgroup's LDS as one
-        single-block kernel; the bits are the same)."""
+        axis at once).  on=2: the same cycle with every pass of the coarse
+        levels in its own launch (the default, True or 1, runs the levels that
+        fit one workgroup's LDS as one single-block kernel; the bits are the
+        same)."""
         _call("dcm_set_precond_multigrid", self.h, 2 if on == 2 else int(bool(on)))
 
     def set_mpdata_variant(self, variant):
@@ -555,6 +556,9 @@ class Model:
         return st
 
     def profile(self, enable=True, only=None):
+        """Per-kernel timing of the next steps: one stream, no graphs, and one
+        launch per pass in a small system's solve, which untimed runs groups
+        of sweeps."""
         _call("dcm_model_profile", self.h, int(enable))
         _call("dcm_model_profile_filter", self.h, only.encode() if only else None)
 

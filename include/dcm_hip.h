@@ -124,10 +124,10 @@ int dcm_fill_along_z(dcm_ctx *ctx, double *a, double lbc, double ubc);
  * inner solve runs an FP32 V-cycle (its outer FP64 refinement still ends
  * every solve at the requested true residual), or, on a grid of constant
  * spacings whose axes have only the factors 2, 3, 5 and 7 and halve together
- * on every level, to two cells or more on the coarsest, applies the operator's inverse itself by Hartley and cosine
- * transforms in the V-cycle's place; the FP64 BiCGSTAB runs the V-cycle in
- * FP64, which is no longer the reference's arithmetic but
- * measures the precision gain at an equal preconditioner.  DCM_BAD_ARG (and
+ * on every level, to two cells or more on the coarsest, applies the
+ * operator's inverse itself by Hartley and cosine transforms in the V-cycle's
+ * place; the FP64 BiCGSTAB runs the V-cycle in FP64, which is no longer the
+ * reference's arithmetic but measures the precision gain beside it.  DCM_BAD_ARG (and
  * no change) when the grid has at most 1024 cells or its dimensions are all
  * odd above 1024 cells.  Off by default.  In a DCM_MIXED ensemble either
  * every member has the setting (each member is then solved with its own
@@ -367,8 +367,11 @@ int dcm_model_field(dcm_model *m, int field, int index, double **dptr);
 int dcm_model_init(dcm_model *m);
 /* Advance nsteps time steps; stats may be NULL. */
 int dcm_model_step(dcm_model *m, int nsteps, dcm_step_stats *stats);
-/* Average kernel time (ms) of the named kernel over the last timed region,
- * and the number of launches it had; returns DCM_BAD_ARG if unknown. */
+/* Per-kernel timing of the following steps on or off (dcm_model_kernel_time
+ * reads it).  While it is on, every kernel is launched by itself on one
+ * stream, without graphs, and a small system is solved with one launch per
+ * pass, as larger ones are, instead of groups of sweeps: the results are the
+ * same bits, but the launches are not all those of an untimed step. */
 int dcm_model_profile(dcm_model *m, int enable);
 /* Time only the kernel groups named in `name`, a comma-separated list
  * (NULL or "": every group). */
@@ -545,6 +548,8 @@ int dcm_output_destroy(dcm_output *o);
 /* ---------------------------------------------------------------------- */
 int dcm_stream_copy(dcm_ctx *ctx, double *dst, const double *src, size_t n,
                     double *ms);
+/* Average kernel time (ms) of the named kernel over the last timed region,
+ * and the number of launches it had; returns DCM_BAD_ARG if unknown. */
 int dcm_model_kernel_time(dcm_model *m, const char *name, double *avg_ms,
                           int *launches);
 
